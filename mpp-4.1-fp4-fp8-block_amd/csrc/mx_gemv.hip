@@ -435,7 +435,10 @@ static hipError_t launch_single(int dual, bool pair, const GemvArgs& g, hipStrea
 // redundant loads when K is short.  The single (down) GEMV takes two row
 // groups per workgroup from 4 tokens on, where x (T x K) staging is large:
 // x is then staged once for 32 rows (measured at C1 with HBM-cold weights:
-// 5.20 -> 5.11 us at T = 8, but 4.3 -> 4.5 us at T = 1).  The dual gate/up
+// 5.20 -> 5.11 us at T = 8, but 4.3 -> 4.5 us at T = 1), where at least 144
+// workgroups remain (N = 2048, K = 5632, T = 8: 64 workgroups 8.9 us, 128 6.7;
+// N = 1024, K = 4096, T = 8: 32 workgroups 6.3 us, 64 4.8; but the MLP of 5760
+// x 5760 at T = 7: 180 workgroups 23.9 us, 360 26.6).  The dual gate/up
 // GEMV keeps one group: its 256 workgroups would halve to 128, idling CUs
 // (measured at C1 T = 8: gate/up 7.0 -> 9.2 us with two groups).
 // Scale planes that are 16-byte aligned (the library's own allocations are)
@@ -443,7 +446,7 @@ static hipError_t launch_single(int dual, bool pair, const GemvArgs& g, hipStrea
 // which are staged in dwords.
 hipError_t launch_gemv_mxfp4(int dual, const GemvArgs& g, hipStream_t st) {
   if (gemv_lds_bytes(g.t, g.k) > 160 * 1024 || g.k > 16384 || g.k % kStepK) return hipErrorInvalidValue;
-  const bool pair = !dual && g.t >= 4 && (g.n / 16) % 2 == 0 && g.k <= 8192 &&
+  const bool pair = !dual && g.t >= 4 && g.n / 16 >= 288 && (g.n / 16) % 2 == 0 && g.k <= 8192 &&
                     gemv_lds_bytes(g.t, g.k, 2) <= 160 * 1024;
   const uintptr_t sp = reinterpret_cast<uintptr_t>(g.s0) | (dual ? reinterpret_cast<uintptr_t>(g.s1) : 0);
   return sp % 16 == 0 ? launch_single<true>(dual, pair, g, st) : launch_single<false>(dual, pair, g, st);
