@@ -45,6 +45,7 @@
 
 #include "mx_device.h"
 #include "mx_internal.h"
+#include "mx_widen.h"
 
 namespace mx {
 namespace qgemm {
@@ -86,62 +87,6 @@ __device__ __forceinline__ void dma4(const void* src, void* lds) {
 constexpr int wait_vm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 // s_waitcnt lgkmcnt(0) alone (vmcnt 63, expcnt 7).
 constexpr int kWaitLgkm0 = 15 | (3 << 14) | (7 << 4);
-
-// INT8 x8 -> f16 x8 (exact): byte b -> half(1024 + (b ^ 0x80)) - 1152.
-__device__ __forceinline__ v8h i8x8_to_f16(uint32_t w0, uint32_t w1) {
-  const uint32_t x[2] = {w0 ^ 0x80808080u, w1 ^ 0x80808080u};
-  v8h out;
-#pragma unroll
-  for (int t = 0; t < 2; t++) {
-    const uint32_t lo = __builtin_amdgcn_perm(0x64646464u, x[t], 0x04010400u);  // b0, b1
-    const uint32_t hi = __builtin_amdgcn_perm(0x64646464u, x[t], 0x04030402u);  // b2, b3
-    v2h l = __builtin_bit_cast(v2h, lo) - (v2h){(_Float16)1152.0f, (_Float16)1152.0f};
-    v2h h = __builtin_bit_cast(v2h, hi) - (v2h){(_Float16)1152.0f, (_Float16)1152.0f};
-    out[4 * t] = l[0]; out[4 * t + 1] = l[1]; out[4 * t + 2] = h[0]; out[4 * t + 3] = h[1];
-  }
-  return out;
-}
-
-// INT4 x8 (one dword, low nibble first) -> f16 x8: ((n ^ 8) - 8) * scale,
-// rounded once to f16 (PackedNumericKernels.metal:30-33).  Per nibble pair
-// (byte i): one v_perm puts byte i of w and of w >> 4 into the two halves,
-// one v_bitop3 keeps their low nibbles, flips the sign bit (two's
-// complement -> offset 8) and ORs in the 0x6400 exponent (1024 + u), then
-// a packed subtract and the packed scale multiply: 17 VALU per dword.
-__device__ __forceinline__ v8h i4x8_to_f16(uint32_t w, _Float16 sc) {
-  const uint32_t y = w >> 4;
-  const v2h off = {(_Float16)1032.0f, (_Float16)1032.0f};
-  const v2h s2 = {sc, sc};
-  v8h out;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const uint32_t t = __builtin_amdgcn_perm(y, w, 0x0c000c00u | (uint32_t)i | ((uint32_t)(4 + i) << 16));
-    const uint32_t p = ((t ^ 0x00080008u) & 0x000f000fu) | 0x64006400u;
-    const v2h q = (__builtin_bit_cast(v2h, p) - off) * s2;
-    out[2 * i] = q[0];
-    out[2 * i + 1] = q[1];
-  }
-  return out;
-}
-
-template <int BK>
-__device__ __forceinline__ v8h fp8x8_to_f16(uint32_t w0, uint32_t w1) {
-  const uint32_t w[2] = {w0, w1};
-  v8h h;
-#pragma unroll
-  for (int t = 0; t < 2; t++) {
-    v2h lo, hi;
-    if (BK == BK_E4M3) {
-      lo = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[t], 1.0f, false);
-      hi = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[t], 1.0f, true);
-    } else {
-      lo = __builtin_amdgcn_cvt_scalef32_pk_f16_bf8(w[t], 1.0f, false);
-      hi = __builtin_amdgcn_cvt_scalef32_pk_f16_bf8(w[t], 1.0f, true);
-    }
-    h[4 * t] = lo[0]; h[4 * t + 1] = lo[1]; h[4 * t + 2] = hi[0]; h[4 * t + 3] = hi[1];
-  }
-  return h;
-}
 
 // One output element's epilogue.  g (and u for SwiGLU) are the raw sums.
 template <int EPI>
@@ -1393,6 +1338,7 @@ bool gemm_q_ok(int ak, int bk, int epi, int m, int n, int k) {
 // MoE form: MXFP4 weights, f16 activations, SwiGLU (mid f16) or f16 store.
 hipError_t launch_gemm_q_grouped(int epi, const QGemmArgs& g, const GroupTable& gt, int groups, hipStream_t st) {
   if (groups < 1 || groups > kMaxGroups || !gemm_q_ok(AK_F16, BK_MXFP4, epi, g.m, g.n, g.k)) return hipErrorInvalidValue;
+  if (stream_wins_grouped(epi, g.n, g.k, gt, groups)) return launch_stream_grouped(epi, g, gt, groups, st);
   switch (epi) {
     case EPI_SWIGLU_F16: return launch_q_grouped<AK_F16, BK_MXFP4, EPI_SWIGLU_F16, 2>(g, gt, groups, st);
     case EPI_STORE_F16:
@@ -1406,9 +1352,13 @@ hipError_t launch_gemm_q(int ak, int bk, int epi, const QGemmArgs& g, hipStream_
   if (!gemm_q_ok(ak, bk, epi, g.m, g.n, g.k)) return hipErrorInvalidValue;
   // few tiles (C0): one small tile per CU, operands requested up front
   // (its scale loads are dwords: planes at a 4-byte boundary)
-  if (ak == AK_F16 && bk == BK_MXFP4 && small_gemm_ok(epi, g.m, g.n, g.k) &&
+  // from 33 rows on (plain GEMMs 17: their 16-row tiles): 16 rows, 1024 -> 2 x
+  // 4096 -> 1024, streaming 4.1 + 5.5 us against 4.7 + 7.5; 64 rows 7.0 + 6.6
+  // against 6.7 + 5.1
+  if (ak == AK_F16 && bk == BK_MXFP4 && small_gemm_ok(epi, g.m, g.n, g.k) && g.m > (is_dual(epi) ? 32 : 16) &&
       ((reinterpret_cast<uintptr_t>(g.s0) | reinterpret_cast<uintptr_t>(g.s1)) & 3u) == 0)
     return launch_small_gemm(epi, g, st);
+  if (stream_wins(ak, bk, epi, g.m, g.n, g.k)) return launch_stream(ak, bk, epi, g, st);
   // about one 64 x 64-channel gate/up tile per CU over a long K (C2): K
   // split between the waves of a workgroup, no split-K partials
   if (bk == BK_MXFP4 && kq_gemm_ok(ak, epi, g.m, g.n, g.k) &&

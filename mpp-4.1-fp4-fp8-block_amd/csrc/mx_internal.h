@@ -109,6 +109,16 @@ struct QGemmArgs {
   const void* pf = nullptr;
   int pf_rows = 0, pf_row_bytes = 0;
 };
+// Weight-streaming GEMM (mx_gemm_stream.h, choice in mx_stream.cpp): any n,
+// k % 32 == 0, few rows (or sizes off the tile grid).  stream_wins: against
+// the 64-K-stage family for a shape that it takes; stream_wins_off_grid:
+// against the K-step-32 kernel; stream_wins_grouped: MoE (g.m = the largest
+// group's rows).
+bool stream_wins(int akind, int bkind, int epi, int m, int n, int k);
+bool stream_wins_off_grid(int akind, int bkind, int epi, int m, int n, int k);
+bool stream_wins_grouped(int epi, int n, int k, const GroupTable& gt, int groups);
+hipError_t launch_stream(int akind, int bkind, int epi, const QGemmArgs& g, hipStream_t st);
+hipError_t launch_stream_grouped(int epi, const QGemmArgs& g, const GroupTable& gt, int groups, hipStream_t st);
 bool gemm_q_ok(int akind, int bkind, int epi, int m, int n, int k);
 size_t gemm_q_ws_bytes(int akind, int bkind, int epi, int m, int n, int k);
 int gemm_q_splits(int akind, int bkind, int epi, int m, int n, int k);
