@@ -1,0 +1,100 @@
+// mx_tile.cpp - which GEMMs the prefill tile kernel (mx_gemm_tile.h) takes, and
+// with which tile.
+#include "mx_tile.h"
+
+#include <algorithm>
+#include <cstdint>
+
+namespace mx {
+
+namespace {
+
+bool dual(int epi) { return epi == EPI_SWIGLU_F16 || epi == EPI_SWIGLU_HALF || epi == EPI_SWIGLU_F32; }
+bool bits4(int bk) { return bk == BK_MXFP4 || bk == BK_INT4G32; }
+long ceil_div(long a, long b) { return (a + b - 1) / b; }
+
+// What the kernel can run: whole rings of K stages, offsets in 32 bits.
+bool can(int ak, int bk, int epi, int k) {
+  if (k > (1 << 20) || epi == EPI_SWIGLU_F8X2) return false;
+  if (ak == AK_I8) return bk == BK_I8 && k % 256 == 0;
+  if (ak != AK_F16 || bk == BK_I8 || epi == EPI_SWIGLU_F32 || epi == EPI_STORE_I32) return false;
+  return k % (bits4(bk) ? 256 : bk == BK_F16 ? 128 : 64) == 0;
+}
+
+bool aligned(int bk, const QGemmArgs& g) {
+  const uintptr_t p = reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b0) | reinterpret_cast<uintptr_t>(g.b1);
+  const uintptr_t s = reinterpret_cast<uintptr_t>(g.s0) | reinterpret_cast<uintptr_t>(g.s1);
+  return p % 16 == 0 && s % (bk == BK_MXFP4 ? 8 : bk == BK_INT4G32 ? 16 : 4) == 0;
+}
+
+// Times of the three kernels, us, per K stage (64 K; int8 128) and for the
+// launch with its first loads and last stores.  The 256-tile runs one workgroup
+// a CU: a full round of 256 costs `full` a stage (the card's matrix rate), one
+// of few tiles `part` (a CU's own).  The 128-tile runs two a CU, so tiles count
+// as fractions of a round, from one tile's own time on.  `tiled`: the 128-row
+// tiles of mx_gemm_q.hip (`start` + `tiled` a stage and round; `deep` at 192 to
+// 256 tiles, where most formats have their deep ring).
+struct Rates {
+  double start256, part, full;
+  double own128, round128;
+  double start, tiled, deep;
+};
+const Rates& rates(int ak, int bk) {
+  static const Rates mxfp4{8, 1.0, 1.46, 0.42, 0.46, 8, 0.535, 0.54};
+  static const Rates int4{10, 1.05, 1.82, 0.55, 0.565, 8, 0.59, 0.6};
+  static const Rates bits8{14, 0.9, 1.54, 0.48, 0.456, 7, 0.5, 0.45};
+  static const Rates f16{8, 0.95, 1.65, 0.58, 0.47, 12, 0.535, 0.55};
+  static const Rates w8a8{19, 1.35, 1.95, 0, 0, 16, 0.61, 0.61};
+  return ak == AK_I8 ? w8a8 : bk == BK_MXFP4 ? mxfp4 : bk == BK_INT4G32 ? int4 : bk == BK_F16 ? f16 : bits8;
+}
+
+// Tile side, 0 where the 128-row tiled family is the faster one.  By the times
+// above, fitted to 200 GEMMs of 256 to 4096 rows (5 formats, 4 MLP sizes), which
+// they get right to 10 % or where the sides differ less.  Some of them, us,
+// tiled / 256 / 128:
+//   MXFP4  4096 -> 2 x 14336   500 rows 139 / 105 / 114   1000 257 / 197 / 205   4096 951 / 670 / 801
+//          14336 -> 4096       500 rows 67 / 237 / 92     1000 152 / 238 / 105   4096 484 / 330 / 398
+//          2048 -> 2 x 5632    1000 rows 54 / 48 / 47     2048 92 / 93 / 89      4096 181 / 153 / 168
+//   FP8    2048 -> 2 x 5632    256 rows 35 / 45 / 22      1000 56 / 56 / 53      4096 186 / 168 / 174
+//          5632 -> 2048        1000 rows 35 / 98 / 44     2048 47 / 100 / 50     4096 95 / 109 / 86
+//   INT4   4096 -> 2 x 14336   500 rows 157 / 123 / 148   1000 284 / 231 / 265   4096 1065 / 820 / 1034
+//   f16    4096 -> 14336       256 rows 40 / 76 / 44      500 103 / 79 / 60      4096 486 / 386 / 432
+//   W8A8   4096 -> 2 x 14336   256 rows 52 / 68           500 110 / 72           4096 563 / 478
+//          14336 -> 4096       1000 rows 78 / 175         2048 139 / 181         4096 262 / 200
+// Below 150 tiles of 128 the split-K launches keep more CUs busy than either
+// tile does; from there to 192 they pay for a second launch and the partials.
+int side_of(int ak, int bk, int epi, int m, int n, int k) {
+  if (!can(ak, bk, epi, k)) return 0;
+  const long n_rows = (long)n * (dual(epi) ? 2 : 1);
+  const long t256 = ceil_div(m, 256) * ceil_div(n_rows, 256), t128 = ceil_div(m, 128) * ceil_div(n_rows, 128);
+  if (t128 < 150) return 0;
+  const double kt = k / (ak == AK_I8 ? 128.0 : 64.0), last = (t256 % 256) / 256.0;
+  const Rates& r = rates(ak, bk);
+  const double us256 = r.start256 + kt * (t256 / 256 * r.full + (last > 0 ? r.part + (r.full - r.part) * last : 0));
+  const double us128 = ak == AK_I8 ? us256 + 1 : 7 + kt * std::max(r.own128, r.round128 * t128 / 256);
+  const double tiled = t128 < 192 ? 17 + kt * 0.32 : t128 <= 256 ? 7 + kt * r.deep : r.start + kt * r.tiled * t128 / 256;
+  return tiled <= std::min(us256, us128) ? 0 : us256 <= us128 ? 256 : 128;
+}
+
+}  // namespace
+
+bool tile_gemm_wins(int ak, int bk, int epi, const QGemmArgs& g) {
+  return aligned(bk, g) && side_of(ak, bk, epi, g.m, g.n, g.k) != 0;
+}
+
+hipError_t launch_tile_gemm(int ak, int bk, int epi, const QGemmArgs& g, hipStream_t st) {
+  using namespace tile;
+  const int side = side_of(ak, bk, epi, g.m, g.n, g.k);
+  if (ak == AK_I8) return launch_i8(epi, g, st);
+  switch (bk) {
+    case BK_MXFP4: return launch_mxfp4(side, epi, g, st);
+    case BK_INT4G32: return launch_int4(side, epi, g, st);
+    case BK_E4M3: return launch_e4m3(side, epi, g, st);
+    case BK_E5M2: return launch_e5m2(side, epi, g, st);
+    case BK_INT8: return launch_int8(side, epi, g, st);
+    case BK_F16: return launch_f16(side, epi, g, st);
+  }
+  return hipErrorInvalidValue;
+}
+
+}  // namespace mx
