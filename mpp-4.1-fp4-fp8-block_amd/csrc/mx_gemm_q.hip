@@ -1366,7 +1366,8 @@ hipError_t launch_gemm_q(int ak, int bk, int epi, const QGemmArgs& g, hipStream_
       ((reinterpret_cast<uintptr_t>(g.s0) | reinterpret_cast<uintptr_t>(g.s1) |
         (ak == AK_F8X2 ? reinterpret_cast<uintptr_t>(g.a_e8) : 0)) & 3u) == 0)
     return launch_kq_gemm(ak, epi, g, st);
-  if (tile_gemm_wins(ak, bk, epi, g)) return launch_tile_gemm(ak, bk, epi, g, st);
+  hipError_t e;
+  if (launch_tile_gemm(ak, bk, epi, g, st, &e)) return e;
   const int s = gemm_q_splits(ak, bk, epi, g.m, g.n, g.k);
   if (s > 1 && !g.ws) return hipErrorInvalidValue;
   if (ak == AK_I8) {

@@ -23,7 +23,9 @@
 // ring in 80 KB, two workgroups a CU.  One barrier a stage, before its last
 // k-step: by then every fragment of the stage is in registers, so its slot is
 // free, and the next stage's fragments are read past it.  Each slot is an array
-// of its own, which is how the compiler's waits tell them apart.
+// of its own, which is how the compiler's waits tell them apart.  Any n, and K in
+// steps of 32: what lies past a row or past K reads as zero, by the DMA's range
+// check.
 //
 // Measured, us, gate/up + down, 128-row tiles of mx_gemm_q.hip -> here, 4096
 // tokens 4096 -> 2 x 14336 -> 4096: MXFP4 951 + 484 -> 670 + 330, E4M3 889 + 450
@@ -89,7 +91,7 @@ __global__ __launch_bounds__(T * 2, 2) void k_tile(QGemmArgs g, int n_tiles) {
   const int tid = threadIdx.x, lane = tid & 63, r32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;
-  const int M = g.m, N = g.n, K = g.k, KT = K / KS;
+  const int M = g.m, N = g.n, K = g.k, KT = (K + KS - 1) / KS;
   const int MT = g.tiles_m;
   // an XCD takes a contiguous run of tiles, walked as 8 weight tiles x all row tiles
   const int tiles = MT * n_tiles, bid = blockIdx.x;
@@ -107,17 +109,24 @@ __global__ __launch_bounds__(T * 2, 2) void k_tile(QGemmArgs g, int n_tiles) {
   const int bfirst = DUAL ? n0 + (wave & (NW / 2 - 1)) * RW : n0 + wave * RW;
   const uint8_t* bsrc = reinterpret_cast<const uint8_t*>(DUAL && wave >= NW / 2 ? g.b1 : g.b0) + (size_t)min(bfirst, N - 1) * b_row;
   const v4i brs = rsrc_of(bsrc, (uint32_t)max(0, min(RW, N - bfirst)) * (uint32_t)b_row);
-  int a_off[NA], b_off[NBI];
+  // (K % 64 == 32: the upper half of the last stage reads as zero too)
+  constexpr int kPast = 0x40000000;  // past every row range
+  const int half_stage = K % KS ? KT - 1 : -1;
+  int a_off[NA], b_off[NBI], a_up[NA], b_up[NBI];
 #pragma unroll
   for (int q = 0; q < NA; q++) {
     const int r = wave * RW + q * 8 + lane / 8;
-    a_off[q] = r * a_row + (((lane % 8) ^ swz<RA>(r)) << 4);
+    const int c = (lane % 8) ^ swz<RA>(r);
+    a_off[q] = r * a_row + (c << 4);
+    a_up[q] = c >= 4 ? kPast : 0;
   }
   constexpr int CB = RB / 16;
 #pragma unroll
   for (int q = 0; q < NBI; q++) {
     const int r = q * (1024 / RB) + lane / CB;   // within the wave's rows
-    b_off[q] = r * b_row + (((lane % CB) ^ swz<RB>(wave * RW + r)) << 4);
+    const int c = (lane % CB) ^ swz<RB>(wave * RW + r);
+    b_off[q] = r * b_row + (c << 4);
+    b_up[q] = c >= CB / 2 ? kPast : 0;
   }
   auto slot = [&](auto u) -> uint8_t* {
     constexpr int U = decltype(u)::value;
@@ -128,13 +137,15 @@ __global__ __launch_bounds__(T * 2, 2) void k_tile(QGemmArgs g, int n_tiles) {
   };
   auto issue = [&](int k, auto u) {
     uint8_t* s = slot(u);
-    const int ao = k < KT ? k * RA : 0x40000000, bo = k < KT ? k * RB : 0x40000000;
+    const int ao = k < KT ? k * RA : kPast, bo = k < KT ? k * RB : kPast, up = k == half_stage ? kPast : 0;
 #pragma unroll
     for (int q = 0; q < NA; q++)
-      llvm_amdgcn_raw_buffer_load_lds_b(ars, (lds_u32)(s + (wave * NA + q) * 1024), 16, a_off[q] + ao, 0, 0, 0);
+      llvm_amdgcn_raw_buffer_load_lds_b(ars, (lds_u32)(s + (wave * NA + q) * 1024), 16,
+                                        a_off[q] + ao + (a_up[q] & up), 0, 0, 0);
 #pragma unroll
     for (int q = 0; q < NBI; q++)
-      llvm_amdgcn_raw_buffer_load_lds_b(brs, (lds_u32)(s + BO + (wave * NBI + q) * 1024), 16, b_off[q] + bo, 0, 0, 0);
+      llvm_amdgcn_raw_buffer_load_lds_b(brs, (lds_u32)(s + BO + (wave * NBI + q) * 1024), 16,
+                                        b_off[q] + bo + (b_up[q] & up), 0, 0, 0);
   };
 
   // ---- fragments
@@ -152,19 +163,30 @@ __global__ __launch_bounds__(T * 2, 2) void k_tile(QGemmArgs g, int n_tiles) {
   }
   constexpr int SW = ESZ * 2;  // dwords of a group's scales
   uint32_t scv[NJ][SW], scn[NJ][SW];  // this group's and the next's, by block
+  // (rows of K / 32 scales start at any byte; the last group's load ends with
+  // the row and is shifted down where it is first used: here it would be waited
+  // for)
   auto scales = [&](int grp4, uint32_t (*d)[SW]) {
     if constexpr (S4) {
 #pragma unroll
-      for (int j = 0; j < NJ; j++) {
-        const uint8_t* s = sc_src[j] + (size_t)min(grp4, KT / 4 - 1) * (8 * ESZ);
-        if constexpr (ESZ == 1) {
-          const v2i v = *reinterpret_cast<const v2i*>(s);
-          d[j][0] = v[0]; d[j][1] = v[1];
-        } else {
-          const v4i v = *reinterpret_cast<const v4i*>(s);
-          d[j][0] = v[0]; d[j][1] = v[1]; d[j][SW > 2 ? 2 : 0] = v[2]; d[j][SW > 2 ? 3 : 0] = v[3];
+      for (int j = 0; j < NJ; j++) __builtin_memcpy(d[j], sc_src[j] + min(grp4 * (8 * ESZ), K / 32 * ESZ - 8 * ESZ), 8 * ESZ);
+    }
+  };
+  auto to_scv = [&](int grp4) {
+    const int sh = max(grp4 * 8 - (K / 32 - 8), 0) * (8 * ESZ);
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+      uint64_t v[ESZ];
+      __builtin_memcpy(v, scn[j], 8 * ESZ);
+      if constexpr (ESZ == 2) {
+        if (sh) {
+          v[0] = sh >= 64 ? v[ESZ - 1] >> (sh & 63) : v[0] >> sh | v[ESZ - 1] << (64 - sh);
+          v[ESZ - 1] = sh >= 64 ? 0 : v[ESZ - 1] >> sh;
         }
+      } else {
+        v[0] >>= sh;
       }
+      __builtin_memcpy(scv[j], v, 8 * ESZ);
     }
   };
   // (the swizzles depend on row % 32 only: one lane part per k-step, constants
@@ -195,7 +217,7 @@ __global__ __launch_bounds__(T * 2, 2) void k_tile(QGemmArgs g, int n_tiles) {
 
   issue(0, std::integral_constant<int, 0>{});
   __builtin_amdgcn_sched_barrier(0);
-  scales(0, scv);
+  scales(0, scn);
   __builtin_amdgcn_sched_barrier(0);
   issue(1, std::integral_constant<int, 1>{});
   if constexpr (NS > 2) issue(2, std::integral_constant<int, 2>{});
@@ -228,6 +250,7 @@ __global__ __launch_bounds__(T * 2, 2) void k_tile(QGemmArgs g, int n_tiles) {
   v4i af[2][MI], bf[NJ][BR];
   v8h bw[2][NJ];
   read_a(r0, 0, af[0]);
+  if constexpr (S4) to_scv(0);
   read_b(r0, bf);
   if constexpr (AK != AK_I8) {
 #pragma unroll
@@ -274,12 +297,7 @@ __global__ __launch_bounds__(T * 2, 2) void k_tile(QGemmArgs g, int n_tiles) {
             acc[i][j] = (Acc)mfma_f16_32x32x16(__builtin_bit_cast(v8h, a[i]), bw[ks & 1][j], (v16f)acc[i][j]);
         }
       if (ks == 3) {
-        if constexpr (S4 && U == 3) {
-#pragma unroll
-          for (int j = 0; j < NJ; j++)
-#pragma unroll
-            for (int t = 0; t < SW; t++) scv[j][t] = scn[j][t];
-        }
+        if constexpr (S4 && U == 3) to_scv(k / 4 + 1);
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
 #pragma unroll
@@ -308,10 +326,15 @@ __global__ __launch_bounds__(T * 2, 2) void k_tile(QGemmArgs g, int n_tiles) {
     if constexpr (NS > 2) stage(k + 2, I2{});
     if constexpr (NS > 3) stage(k + 3, I3{});
   }
-  if constexpr (NS == 3) {
-    if (k < KT) {
-      stage(k, I0{});
-      if (k + 1 < KT) stage(k + 1, I1{});
+  if (k < KT) {
+    stage(k, I0{});
+    if constexpr (NS > 2) {
+      if (k + 1 < KT) {
+        stage(k + 1, I1{});
+        if constexpr (NS > 3) {
+          if (k + 2 < KT) stage(k + 2, I2{});
+        }
+      }
     }
   }
 
@@ -331,10 +354,7 @@ __global__ __launch_bounds__(T * 2, 2) void k_tile(QGemmArgs g, int n_tiles) {
       uint32_t hit = 0;
 #pragma unroll
       for (int j = 0; j < NJ; j++)
-        for (int t = 0; t < K / 32; t += 4) {
-          const uint32_t c = ~*reinterpret_cast<const uint32_t*>(sc_src[j] + t);  // a zero byte?
-          hit |= (c - 0x01010101u) & ~c & 0x80808080u;
-        }
+        for (int t = 0; t < K / 32; t++) hit |= sc_src[j][t] == 255u;
       if (__ballot(hit != 0) != 0) {
         const uint8_t* ap[MI];
         const uint8_t* bp[NJ];
@@ -352,13 +372,21 @@ __global__ __launch_bounds__(T * 2, 2) void k_tile(QGemmArgs g, int n_tiles) {
         }
 #pragma unroll 1
         for (int t = 0; t < KT * 4; t++) {  // k-step t % 4 of stage t / 4
+          const bool in = (t >> 2) * 64 + h * 32 < K;
           v4i a[MI];
 #pragma unroll
-          for (int i = 0; i < MI; i++) a[i] = *reinterpret_cast<const v4i*>(ap[i] + (t >> 2) * RA + (t & 3) * 16);
+          for (int i = 0; i < MI; i++) {
+            a[i] = v4i{0, 0, 0, 0};
+            if (in) a[i] = *reinterpret_cast<const v4i*>(ap[i] + (t >> 2) * RA + (t & 3) * 16);
+          }
 #pragma unroll
           for (int j = 0; j < NJ; j++) {
-            const uint32_t w = *reinterpret_cast<const uint32_t*>(bp[j] + t / 4 * RB + t % 4 * 4);
-            const v8h b = fp4x8_dequant_f16(w, sc_src[j][t / 4 * 2 + h]);
+            uint32_t w = 0, sb = 0;
+            if (in) {
+              w = *reinterpret_cast<const uint32_t*>(bp[j] + t / 4 * RB + t % 4 * 4);
+              sb = sc_src[j][t / 4 * 2 + h];
+            }
+            const v8h b = fp4x8_dequant_f16(w, sb);
 #pragma unroll
             for (int i = 0; i < MI; i++) acc[i][j] = mfma_f16_32x32x16(__builtin_bit_cast(v8h, a[i]), b, acc[i][j]);
           }

@@ -109,10 +109,11 @@ struct QGemmArgs {
   const void* pf = nullptr;
   int pf_rows = 0, pf_row_bytes = 0;
 };
-// Prefill tile GEMM (mx_gemm_tile.h, choice in mx_tile.cpp) against the
-// 64-K-stage family, for a shape that it takes.
-bool tile_gemm_wins(int akind, int bkind, int epi, const QGemmArgs& g);
-hipError_t launch_tile_gemm(int akind, int bkind, int epi, const QGemmArgs& g, hipStream_t st);
+// Prefill tile GEMM (mx_gemm_tile.h, choice in mx_tile.cpp): launched, with its
+// status in *e, where it is faster than the 64-K-stage family (off_grid: than
+// the kernels for sizes off the 64-wide grid); false where it is not.
+bool launch_tile_gemm(int akind, int bkind, int epi, const QGemmArgs& g, hipStream_t st, hipError_t* e);
+bool launch_tile_gemm_off_grid(int akind, int bkind, int epi, const QGemmArgs& g, hipStream_t st, hipError_t* e);
 // Weight-streaming GEMM (mx_gemm_stream.h, choice in mx_stream.cpp): any n,
 // k % 32 == 0, few rows (or sizes off the tile grid).  stream_wins: against
 // the 64-K-stage family for a shape that it takes; stream_wins_off_grid:

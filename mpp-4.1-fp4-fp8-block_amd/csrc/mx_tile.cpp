@@ -13,18 +13,18 @@ bool dual(int epi) { return epi == EPI_SWIGLU_F16 || epi == EPI_SWIGLU_HALF || e
 bool bits4(int bk) { return bk == BK_MXFP4 || bk == BK_INT4G32; }
 long ceil_div(long a, long b) { return (a + b - 1) / b; }
 
-// What the kernel can run: whole rings of K stages, offsets in 32 bits.
+// What the kernel can run: a whole group of scales, offsets in 32 bits.
 bool can(int ak, int bk, int epi, int k) {
   if (k > (1 << 20) || epi == EPI_SWIGLU_F8X2) return false;
-  if (ak == AK_I8) return bk == BK_I8 && k % 256 == 0;
+  if (ak == AK_I8) return bk == BK_I8 && k % 128 == 0;
   if (ak != AK_F16 || bk == BK_I8 || epi == EPI_SWIGLU_F32 || epi == EPI_STORE_I32) return false;
-  return k % (bits4(bk) ? 256 : bk == BK_F16 ? 128 : 64) == 0;
+  return k % 32 == 0 && k >= 256;
 }
 
 bool aligned(int bk, const QGemmArgs& g) {
   const uintptr_t p = reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b0) | reinterpret_cast<uintptr_t>(g.b1);
   const uintptr_t s = reinterpret_cast<uintptr_t>(g.s0) | reinterpret_cast<uintptr_t>(g.s1);
-  return p % 16 == 0 && s % (bk == BK_MXFP4 ? 8 : bk == BK_INT4G32 ? 16 : 4) == 0;
+  return p % 16 == 0 && s % (bk == BK_MXFP4 ? 1 : bk == BK_INT4G32 ? 2 : 4) == 0;
 }
 
 // Times of the three kernels, us, per K stage (64 K; int8 128) and for the
@@ -48,6 +48,19 @@ const Rates& rates(int ak, int bk) {
   return ak == AK_I8 ? w8a8 : bk == BK_MXFP4 ? mxfp4 : bk == BK_INT4G32 ? int4 : bk == BK_F16 ? f16 : bits8;
 }
 
+struct Times {
+  long t128;
+  double us256, us128;
+};
+Times times(int ak, int bk, int epi, int m, int n, int k) {
+  const long n_rows = (long)n * (dual(epi) ? 2 : 1);
+  const long t256 = ceil_div(m, 256) * ceil_div(n_rows, 256), t128 = ceil_div(m, 128) * ceil_div(n_rows, 128);
+  const double kt = k / (ak == AK_I8 ? 128.0 : 64.0), last = (t256 % 256) / 256.0;
+  const Rates& r = rates(ak, bk);
+  const double us256 = r.start256 + kt * (t256 / 256 * r.full + (last > 0 ? r.part + (r.full - r.part) * last : 0));
+  return {t128, us256, ak == AK_I8 ? us256 + 1 : 7 + kt * std::max(r.own128, r.round128 * t128 / 256)};
+}
+
 // Tile side, 0 where the 128-row tiled family is the faster one.  By the times
 // above, fitted to 200 GEMMs of 256 to 4096 rows (5 formats, 4 MLP sizes), which
 // they get right to 10 % or where the sides differ less.  Some of them, us,
@@ -65,26 +78,30 @@ const Rates& rates(int ak, int bk) {
 // tile does; from there to 192 they pay for a second launch and the partials.
 int side_of(int ak, int bk, int epi, int m, int n, int k) {
   if (!can(ak, bk, epi, k)) return 0;
-  const long n_rows = (long)n * (dual(epi) ? 2 : 1);
-  const long t256 = ceil_div(m, 256) * ceil_div(n_rows, 256), t128 = ceil_div(m, 128) * ceil_div(n_rows, 128);
-  if (t128 < 150) return 0;
-  const double kt = k / (ak == AK_I8 ? 128.0 : 64.0), last = (t256 % 256) / 256.0;
+  const Times t = times(ak, bk, epi, m, n, k);
+  if (t.t128 < 150) return 0;
+  const double kt = k / (ak == AK_I8 ? 128.0 : 64.0);
   const Rates& r = rates(ak, bk);
-  const double us256 = r.start256 + kt * (t256 / 256 * r.full + (last > 0 ? r.part + (r.full - r.part) * last : 0));
-  const double us128 = ak == AK_I8 ? us256 + 1 : 7 + kt * std::max(r.own128, r.round128 * t128 / 256);
-  const double tiled = t128 < 192 ? 17 + kt * 0.32 : t128 <= 256 ? 7 + kt * r.deep : r.start + kt * r.tiled * t128 / 256;
-  return tiled <= std::min(us256, us128) ? 0 : us256 <= us128 ? 256 : 128;
+  const double tiled = t.t128 < 192 ? 17 + kt * 0.32 : t.t128 <= 256 ? 7 + kt * r.deep : r.start + kt * r.tiled * t.t128 / 256;
+  return tiled <= std::min(t.us256, t.us128) ? 0 : t.us256 <= t.us128 ? 256 : 128;
+}
+
+// Sizes off the 64-wide grid: against streaming at 330 (4-bit) or 250 TFLOP/s
+// (mx_stream.cpp); the K-step-32 kernel is slower than one of the two.  us, the
+// faster of those -> here: MXFP4 MLPs of 1374 tokens, 2336 -> 13472, 711 -> 282;
+// 1126 tokens, 1888 -> 5248, 139 -> 83; 2685 tokens, 2144 -> 4736, 361 -> 168; FP8
+// 455 tokens, 5920 -> 6048, 294 -> 147; 1796 x 2560 x 2208 69 -> 36.
+int side_off_grid(int ak, int bk, int epi, int m, int n, int k) {
+  if (ak != AK_F16 || !can(ak, bk, epi, k)) return 0;
+  const Times t = times(ak, bk, epi, m, n, k);
+  const double stream = 5 + 2.0 * m * n * (dual(epi) ? 2 : 1) * k / (bits4(bk) ? 3.3e8 : 2.5e8);
+  return stream <= std::min(t.us256, t.us128) ? 0 : t.us256 <= t.us128 ? 256 : 128;
 }
 
 }  // namespace
 
-bool tile_gemm_wins(int ak, int bk, int epi, const QGemmArgs& g) {
-  return aligned(bk, g) && side_of(ak, bk, epi, g.m, g.n, g.k) != 0;
-}
-
-hipError_t launch_tile_gemm(int ak, int bk, int epi, const QGemmArgs& g, hipStream_t st) {
+static hipError_t launch_side(int side, int ak, int bk, int epi, const QGemmArgs& g, hipStream_t st) {
   using namespace tile;
-  const int side = side_of(ak, bk, epi, g.m, g.n, g.k);
   if (ak == AK_I8) return launch_i8(epi, g, st);
   switch (bk) {
     case BK_MXFP4: return launch_mxfp4(side, epi, g, st);
@@ -95,6 +112,18 @@ hipError_t launch_tile_gemm(int ak, int bk, int epi, const QGemmArgs& g, hipStre
     case BK_F16: return launch_f16(side, epi, g, st);
   }
   return hipErrorInvalidValue;
+}
+
+bool launch_tile_gemm(int ak, int bk, int epi, const QGemmArgs& g, hipStream_t st, hipError_t* e) {
+  const int side = aligned(bk, g) ? side_of(ak, bk, epi, g.m, g.n, g.k) : 0;
+  if (side) *e = launch_side(side, ak, bk, epi, g, st);
+  return side != 0;
+}
+
+bool launch_tile_gemm_off_grid(int ak, int bk, int epi, const QGemmArgs& g, hipStream_t st, hipError_t* e) {
+  const int side = aligned(bk, g) ? side_off_grid(ak, bk, epi, g.m, g.n, g.k) : 0;
+  if (side) *e = launch_side(side, ak, bk, epi, g, st);
+  return side != 0;
 }
 
 }  // namespace mx

@@ -8,14 +8,16 @@ import pytest
 
 import mxfp4hip as M
 from mlp_data import MlpData
-from test_gpu_stream import close, mxfp4
+from test_gpu_stream import E2M1, close, mxfp4
 
 pytestmark = pytest.mark.gpu
 
 
 # (m, n, k) on the 128- and 256-wide tiles: whole, one row or 64 channels past
-# a tile, one row short, a single 256-K ring
-SHAPES = [(1024, 4096, 256), (1281, 8128, 768), (1000, 4160, 512), (4096, 4096, 512), (4095, 4160, 768), (4097, 2112, 1280)]
+# a tile, one row short, a single 256-K ring; then K that ends a quarter, half or
+# three quarters into a group of four stages, or in the middle of a stage
+SHAPES = [(1024, 4096, 256), (1281, 8128, 768), (1000, 4160, 512), (4096, 4096, 512), (4095, 4160, 768), (4097, 2112, 1280),
+          (1281, 8128, 320), (4095, 4160, 384), (4095, 4160, 448), (1500, 5013, 288), (4095, 4131, 416), (4097, 2099, 1440)]
 
 
 @pytest.mark.parametrize("m,n,k", SHAPES)
@@ -36,9 +38,10 @@ def test_matmul_mxfp4(dev, m, n, k):
         b.free()
 
 
-def test_matmul_e8m0_255(dev):
+@pytest.mark.parametrize("k", [512, 800, 1376])
+def test_matmul_e8m0_255(dev, k):
     """Byte 255 is +inf: the columns it reaches follow IEEE, the others stand."""
-    m, n, k = 4096, 4160, 512
+    m, n = 4096, 4160
     rng = np.random.default_rng(5)
     q, s, w = mxfp4(rng, n, k)
     a = rng.standard_normal((m, k)).astype(np.float16)
@@ -47,6 +50,8 @@ def test_matmul_e8m0_255(dev):
     cols = [0, 255, 300, 4159]
     for c in cols:
         s[c, 3] = 255
+    s[300, 3], s[300, -1] = 130, 255  # the row's last block
+    w[300] = E2M1[np.stack([q[300] & 15, q[300] >> 4], -1).reshape(k)] * np.repeat(2.0 ** (np.where(s[300] == 255, 127, s[300]).astype(np.float64) - 127), 32)
     q[255, 48:64], w[255, 96:128] = 0x22, 1  # positive codes only: +-inf where the signs of x agree, as in rows 0 to 5
     a[:6] = np.abs(a[:6])
     with np.errstate(invalid="ignore"):
@@ -77,7 +82,7 @@ def test_gemm_f16_weights(dev, m, n, k):
         x.free()
 
 
-@pytest.mark.parametrize("m,n,k", [(4096, 4096, 256), (4095, 4160, 768), (3841, 4160, 1280)])
+@pytest.mark.parametrize("m,n,k", [(4096, 4096, 256), (4095, 4160, 896), (3841, 4160, 1280)])
 def test_gemm_i8_exact(dev, m, n, k):
     rng = np.random.default_rng(m + n + k)
     a = rng.integers(-127, 128, (m, k)).astype(np.int8)
@@ -91,11 +96,13 @@ def test_gemm_i8_exact(dev, m, n, k):
 
 
 @pytest.mark.parametrize("fmt", [0, -1, M.WFMT_FP8_E4M3, M.WFMT_FP8_E5M2, M.WFMT_INT8, M.WFMT_INT4, M.WFMT_W8A8])
-@pytest.mark.parametrize("tokens,h,i", [(1281, 1024, 2816), (4095, 2304, 2304), (2049, 768, 4096)])
+@pytest.mark.parametrize("tokens,h,i", [(1281, 1024, 2816), (4095, 2304, 2304), (2049, 768, 4096), (4095, 1888, 1696)])
 def test_mlp_rows(dev, fmt, tokens, h, i):
     """Rows of a large batch against the same rows alone, which other kernels
     run: f32 sums in another order, so f16 mids and results differ by a step
     (2^-10 relative, results up to 6 rms) at most.  -1: REFROW (f32 result)."""
+    if fmt == M.WFMT_W8A8 and (h % 128 or i % 128):
+        pytest.skip("W8A8 takes multiples of 128")
     d = MlpData(dev, tokens, h, i, seed=tokens + fmt, wfmt=max(fmt, 0))
     out = dev.alloc(tokens * h * 4)
     npdt = np.float32 if fmt < 0 else np.float16
