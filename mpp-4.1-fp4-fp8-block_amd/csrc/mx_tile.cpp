@@ -81,6 +81,10 @@ int side_of(int ak, int bk, int epi, int m, int n, int k) {
   const Times t = times(ak, bk, epi, m, n, k);
   if (t.t128 < 150) return 0;
   const double kt = k / (ak == AK_I8 ? 128.0 : 64.0);
+  // MXFP4 up to one round of tiles and 2048 K: level with the tiled family's deep
+  // ring as a kernel, behind it in a pass (512 rows, 7168 -> 2 x 2048 -> 7168, the
+  // down GEMM here 48.55 us a pass, there 48.07; 4096 K, 256 tiles: 34.2 against 35.0)
+  if (bk == BK_MXFP4 && t.t128 >= 192 && t.t128 <= 256 && kt <= 32) return 0;
   const Rates& r = rates(ak, bk);
   const double tiled = t.t128 < 192 ? 17 + kt * 0.32 : t.t128 <= 256 ? 7 + kt * r.deep : r.start + kt * r.tiled * t.t128 / 256;
   return tiled <= std::min(t.us256, t.us128) ? 0 : t.us256 <= t.us128 ? 256 : 128;
