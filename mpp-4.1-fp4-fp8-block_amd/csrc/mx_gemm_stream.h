@@ -370,6 +370,9 @@ __device__ __forceinline__ void tile(const Args& g, int m0, int nt, const Lds& l
 #pragma unroll
         for (int h = 0; h < NB; h++) w[gi][h] = w2[gi][PS == 2 ? U % PS : h];
       if ((st + 1) * kStep > K) {  // a last step of less than 128 K: zero what is past the end
+        // (the scales too: an infinite one of the row's last block makes a zero code NaN)
+#pragma unroll
+        for (int gi = 0; gi < NG; gi++) s[gi] = st * 4 + lg < KB ? s[gi] : 0u;
 #pragma unroll
         for (int q = 0; q < NQ; q++) {
           const bool in = st * RB + a_chunk(q) * 16 < a_row;

@@ -125,6 +125,34 @@ def test_matmul_byte_255(dev, m, k):
         b.free()
 
 
+@pytest.mark.parametrize("I", [160, 192, 224])
+def test_int4_last_scale_infinite(dev, I):
+    """An infinite f16 scale on a row's last block, where K ends within a
+    128-K step: +-inf where the block's codes have one sign, nowhere else."""
+    T, H = 5, 128
+    d = MlpData(dev, T, H, I, seed=I, wfmt=M.WFMT_INT4)
+    x, mats = d.host()
+    x = np.abs(x) + np.float16(0.1)
+    for q, _ in mats[:2]:
+        q[I - 32:] = 0x11  # the last 32 mid channels are positive
+    qd, sd = mats[2]
+    qd[5, -16:], qd[H - 1, -16:] = 0x11, 0xFF
+    sd[[5, H - 1], -1] = np.inf
+    for host, buf in [(x, d.x)] + [(h, b) for hs, bs in zip(mats, d.mats) for h, b in zip(hs, bs)]:
+        dev.upload(host, buf)
+    out = dev.alloc(T * H * 2)
+    dev.fmt_mlp_forward(M.WFMT_INT4, T, H, I, d.x, d.weights, out)
+    got = dev.download(out, np.float16, (T, H))
+    assert (got[:, 5] == np.inf).all() and (got[:, H - 1] == -np.inf).all(), got[:, [5, H - 1]]
+    keep = np.setdiff1d(np.arange(H), [5, H - 1])
+    sd[[5, H - 1], -1] = 1
+    ref = O.mlp_format(M.WFMT_INT4, x, *mats[0], *mats[1], *mats[2], H, I)
+    rel, cos = O.mlp_error(got[:, keep], ref[:, keep])
+    assert rel <= O.MAX_ABS_REL_TOL and cos >= O.COSINE_TOL, (rel, cos)
+    out.free()
+    d.free()
+
+
 @pytest.mark.parametrize("counts,H,I", [
     ([25, 0, 3, 17, 1, 8, 9, 33], 512, 384),   # 16-row tiles, all tile bodies, an empty group
     ([90, 1, 40, 33], 256, 1152),              # 32-row tiles
