@@ -1337,6 +1337,7 @@ bool gemm_q_ok(int ak, int bk, int epi, int m, int n, int k) {
 
 // MoE form: MXFP4 weights, f16 activations, SwiGLU (mid f16) or f16 store.
 hipError_t launch_gemm_q_grouped(int epi, const QGemmArgs& g, const GroupTable& gt, int groups, hipStream_t st) {
+  if (epi != EPI_SWIGLU_F16 && epi != EPI_STORE_F16) return hipErrorInvalidValue;
   if (groups < 1 || groups > kMaxGroups || !gemm_q_ok(AK_F16, BK_MXFP4, epi, g.m, g.n, g.k)) return hipErrorInvalidValue;
   if (stream_wins_grouped(epi, g.n, g.k, gt, groups)) return launch_stream_grouped(epi, g, gt, groups, st);
   switch (epi) {

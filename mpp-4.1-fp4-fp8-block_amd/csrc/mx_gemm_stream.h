@@ -593,7 +593,7 @@ hipError_t launch_rows(const Args& g, const GroupTable* gt, int groups, int ng, 
   return hipErrorInvalidValue;
 }
 
-// One weight format: tile rows and groups from plan().
+// One weight format: tile rows and groups as launch_stream chose them.
 template <int AK, int BK, bool GROUPED>
 hipError_t launch_bk(const Args& g, const GroupTable* gt, int groups, int rows, int ng, hipStream_t st) {
   switch (rows) {

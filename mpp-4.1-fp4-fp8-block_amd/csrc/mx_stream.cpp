@@ -10,10 +10,6 @@ using namespace stream;
 
 namespace {
 
-struct Plan {
-  int rows, ng;
-};
-
 bool bits4(int bk) { return bk == BK_MXFP4 || bk == BK_INT4G32; }
 
 // Bytes of a workgroup's scale copy.
@@ -81,9 +77,10 @@ Args args_of(int epi, const QGemmArgs& q) {
 // What the kernel can run: its scale copy, and offsets in 32 bits.
 bool can(int ak, int bk, int epi, int n, int k) {
   if (k % 32 || k > (1 << 20) || (size_t)n * (is_dual(epi) ? 2 : 1) > (1u << 30) || scale_bytes(bk, 1, k) > kScales) return false;
-  if (ak == AK_I8) return bk == BK_I8 && k % 128 == 0;
-  if (ak == AK_F32) return (bk == BK_F16 || bk == BK_MXFP4) && !is_dual(epi);
-  return ak == AK_F16 && bk != BK_I8 && epi != EPI_SWIGLU_F8X2 && epi != EPI_STORE_I32 && epi != EPI_SWIGLU_F32;
+  const bool store = epi == EPI_STORE_F32 || epi == EPI_STORE_F16;
+  if (ak == AK_I8) return bk == BK_I8 && k % 128 == 0 && (store || epi == EPI_STORE_I32 || epi == EPI_SWIGLU_F32);
+  if (ak == AK_F32) return (bk == BK_F16 || bk == BK_MXFP4) && store;
+  return ak == AK_F16 && bk != BK_I8 && (store || epi == EPI_SWIGLU_F16 || epi == EPI_SWIGLU_HALF);
 }
 
 }  // namespace
