@@ -81,10 +81,18 @@ int side_of(int ak, int bk, int epi, int m, int n, int k) {
   const Times t = times(ak, bk, epi, m, n, k);
   if (t.t128 < 150) return 0;
   const double kt = k / (ak == AK_I8 ? 128.0 : 64.0);
-  // MXFP4 up to one round of tiles and 2048 K: level with the tiled family's deep
-  // ring as a kernel, behind it in a pass (512 rows, 7168 -> 2 x 2048 -> 7168, the
-  // down GEMM here 48.55 us a pass, there 48.07; 4096 K, 256 tiles: 34.2 against 35.0)
-  if (bk == BK_MXFP4 && t.t128 >= 192 && t.t128 <= 256 && kt <= 32) return 0;
+  // MXFP4, a plain store, one round of tiles, up to 2048 K: level with the tiled
+  // family's deep ring as a kernel (0.8 us faster to 0.8 slower), behind it or
+  // level in a pass.  Down GEMMs of MLP passes, us a pass, deep ring / here: 512
+  // rows, 7168 wide, K = 1024 34.9 / 35.9, 1536 44.4 / 44.9, 2048 50.9 / 51.1, 2560
+  // 79.0 / 79.7; 6656, 1024 38.8 / 40.0; 8192, 1024 38.1 / 39.0; 768 rows, 4608, 1024
+  // 32.3 / 32.8; 1024 rows, 4096, 1024 35.1 / 35.9; 1500 rows, 2304, 2048 47.9 / 48.3;
+  // 1792 rows, 2048, 1536 40.9 / 41.8; 2048 rows, 2048, 2048 50.6 / 51.0; past it 1024
+  // rows, 4096, K = 2560 84.8 / 84.7, 3584 85.9 / 85.7.  Gate/up GEMMs of the same
+  // tiles and K are faster here: 1024 rows, 2048 -> 2 x 2048 41.1 / 39.5, 768 rows,
+  // 2048 -> 2 x 2304 39.1 / 38.2, 900 rows, 2048 -> 2 x 1792 39.7 / 38.7, 512 rows, 2048
+  // -> 2 x 3584 36.6 / 36.0, K = 1024 level.
+  if (bk == BK_MXFP4 && !dual(epi) && t.t128 >= 192 && t.t128 <= 256 && kt <= 32) return 0;
   const Rates& r = rates(ak, bk);
   const double tiled = t.t128 < 192 ? 17 + kt * 0.32 : t.t128 <= 256 ? 7 + kt * r.deep : r.start + kt * r.tiled * t.t128 / 256;
   return tiled <= std::min(t.us256, t.us128) ? 0 : t.us256 <= t.us128 ? 256 : 128;
