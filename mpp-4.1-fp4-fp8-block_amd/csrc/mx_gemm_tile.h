@@ -50,6 +50,16 @@ constexpr int rb_of(int bk) { return bk == BK_F16 || bk == BK_I8 ? 128 : bits4(b
 constexpr int slots_of(int bk) { return rb_of(bk) == 128 ? 2 : bits4(bk) ? 4 : 3; }
 constexpr int wait_lgkm0_vm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
 
+// Scales by which the load of scale group g starts early, so that it ends with
+// the row's n scales (n >= 8).  Groups past the row (read ahead, never used)
+// stay at 7: a shift below the group's width.
+__host__ __device__ constexpr int late_scales(int g, int n) {
+  const int late = g * 8 - (n - 8);
+  return late < 0 ? 0 : late > 7 ? 7 : late;
+}
+static_assert(late_scales(0, 8) == 0 && late_scales(1, 16) == 0 && late_scales(1, 9) == 7 && late_scales(1, 15) == 1, "last group");
+static_assert(late_scales(1, 8) == 7 && late_scales(2, 9) == 7, "past the last group");
+
 // 16-byte chunks of a row are stored at chunk ^ swz(row): the 32 lanes of a
 // fragment read, one row each, then cover all banks.
 template <int R>
@@ -173,7 +183,7 @@ __global__ __launch_bounds__(T * 2, 2) void k_tile(QGemmArgs g, int n_tiles) {
     }
   };
   auto to_scv = [&](int grp4) {
-    const int sh = max(grp4 * 8 - (K / 32 - 8), 0) * (8 * ESZ);
+    const int sh = late_scales(grp4, K / 32) * (8 * ESZ);
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
       uint64_t v[ESZ];
