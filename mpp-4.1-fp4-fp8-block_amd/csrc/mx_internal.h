@@ -114,6 +114,8 @@ struct QGemmArgs {
 // the kernels for sizes off the 64-wide grid); false where it is not.
 bool launch_tile_gemm(int akind, int bkind, int epi, const QGemmArgs& g, hipStream_t st, hipError_t* e);
 bool launch_tile_gemm_off_grid(int akind, int bkind, int epi, const QGemmArgs& g, hipStream_t st, hipError_t* e);
+// Estimate of a GEMM there, us; infinite where launch_tile_gemm does not take it.
+double tile_gemm_time(int akind, int bkind, int epi, int m, int n, int k);
 // Weight-streaming GEMM (mx_gemm_stream.h, choice in mx_stream.cpp): any n,
 // k % 32 == 0, few rows (or sizes off the tile grid).  stream_wins: against
 // the 64-K-stage family for a shape that it takes; stream_wins_off_grid:
@@ -121,6 +123,9 @@ bool launch_tile_gemm_off_grid(int akind, int bkind, int epi, const QGemmArgs& g
 // group's rows).
 bool stream_wins(int akind, int bkind, int epi, int m, int n, int k);
 bool stream_wins_off_grid(int akind, int bkind, int epi, int m, int n, int k);
+// stream_time, k32_time: estimates of it and of the K-step-32 kernel, us.
+double stream_time(int akind, int bkind, int epi, int m, int n, int k);
+double k32_time(int akind, int epi, int m, int n, int k);
 bool stream_wins_grouped(int epi, int n, int k, const GroupTable& gt, int groups);
 hipError_t launch_stream(int akind, int bkind, int epi, const QGemmArgs& g, hipStream_t st);
 hipError_t launch_stream_grouped(int epi, const QGemmArgs& g, const GroupTable& gt, int groups, hipStream_t st);

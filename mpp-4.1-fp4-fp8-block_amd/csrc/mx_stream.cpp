@@ -3,6 +3,7 @@
 #include "mx_stream.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace mx {
 
@@ -85,50 +86,91 @@ bool can(int ak, int bk, int epi, int n, int k) {
 
 }  // namespace
 
-// The tiled family's time is almost flat up to 128 rows (its tile) and set by
-// the latency of its K stages; this kernel's grows with row tiles x weight
-// bytes.  Both sides measured at 1 to 256 rows, us, tiled -> streaming:
+// Rounds that workgroups filling the chip x times take: between x (they start
+// as others end) and whole ones.
+static double rounds_of(double x) { return std::max(1.0, 0.55 * x + 0.45 * std::ceil(x)); }
+
+// Time of a launch, us: 2 for it, its first loads and its sums, and for each
+// workgroup of a CU 0.055 a step and KB and 0.65 (4-bit weights) to 1.5 a group
+// of weight rows for its scales and its outputs; two share a CU, further ones
+// start as one ends.  Or, if that is more, each row tile's read of the weights
+// at 4.6 TB/s.  Fitted to 1700 GEMMs of 17 to 4097 rows, K of 64 to 16384; half
+// of them are within 5 %, nine in ten within 17 %.
+double stream_time(int ak, int bk, int epi, int m, int n, int k) {
+  if (!can(ak, bk, epi, n, k)) return HUGE_VAL;
+  struct Rate { double start, wg, kb, group; };
+  const Rate r = ak == AK_I8 ? Rate{2.8, -1.8, 0.05, 1.45} : ak == AK_F32 ? Rate{1.9, 0.3, 0.055, 0.9}
+                 : bits4(bk) ? Rate{2.3, 0, 0.055, 0.65} : bk == BK_F16 ? Rate{1.5, 0.3, 0.052, 1.2} : Rate{2.1, 0, 0.058, 0.9};
+  const int rows = tile_rows(ak, m), tiles = (m + rows - 1) / rows;
+  const int ng = groups_of(ak, bk, epi, rows, n, k, tiles);
+  const double f = fill(epi, n, ng, tiles), kb = 8 + ng * (bits4(bk) ? 2 : bk == BK_F16 ? 8 : 4);
+  const double wg = r.wg + r.kb * (k / 512.0) * kb + r.group * ng;
+  const double rounds = f > 2 ? (f + std::ceil(f)) / 2 : f > 1 ? 1.84 : 0.92;
+  return std::max(2.5 + tiles * weight_mb(bk, epi, n, k) / 4.6, r.start + std::max(0.3, rounds * wg));
+}
+
+// Time of the 64-K-stage family, us (1700 GEMMs of its sizes, half within 8 %,
+// nine in ten within 25 %): rounds of 256 workgroups at 0.5 a K stage (f32
+// activations 1.35), a split's partials at 2.1 MB a us and their sum, the weights
+// at 3.3 TB/s (W8A8 4.6).
+static double tiled_time(int ak, int bk, int epi, int m, int n, int k) {
+  struct Rate { double start, stage, round, split; };
+  const Rate r = ak == AK_F32 ? Rate{0.7, 1.35, 3.05, 2.5} : ak == AK_I8 ? Rate{1.6, 0.49, 3.9, 2.5}
+                 : bk == BK_F16 ? Rate{1.6, 0.43, 1.35, 1.65} : bk == BK_INT4G32 ? Rate{1.75, 0.635, 1.65, 1.65}
+                 : bk == BK_MXFP4 ? Rate{1.5, 0.52, 1.6, 2.0} : Rate{3.7, 0.5, 0.85, 0.35};
+  const int s = gemm_q_splits(ak, bk, epi, m, n, k);
+  const long tiles = (long)((m + 127) / 128) * (!is_dual(epi) && n % 128 == 0 ? n / 128 : n / 64);
+  double t = r.start + (r.stage * k / (ak == AK_I8 ? 128 : 64) / s + r.round) * rounds_of(tiles * s / 256.0);
+  if (s > 1) t += r.split + 0.47 * s * (is_dual(epi) ? 2 : 1) * m * n * 4e-6 + (ak == AK_I8 ? 0 : 0.27 * s);
+  // MXFP4 gate/up from HBM: a tenth more (76 rows, 3072 -> 2 x 3072: 17.0 us)
+  if (bk == BK_MXFP4 && is_dual(epi)) t *= 1.1;
+  // one 64 x 64-channel gate/up tile per CU (34 rows, 2560 -> 2 x 12416: 14.1
+  // us against 26.0 streaming; 512 rows, 7168 -> 2 x 2048: 31)
+  if (bk == BK_MXFP4 && kq_gemm_ok(ak, epi, m, n, k)) t = std::min(t, 4.7 + 0.0037 * k);
+  return std::max(t, weight_mb(bk, epi, n, k) / (ak == AK_I8 ? 4.6 : 3.3));
+}
+
+// Time of the K-step-32 kernel, us, of 64 columns x 64 rows a workgroup, or 128
+// rows from 256 such workgroups on (390 GEMMs off the grid, 2 to 4000 rows, half
+// within 12 %).
+double k32_time(int ak, int epi, int m, int n, int k) {
+  const long cols = (n + 63) / 64, w128 = cols * ((m + 127) / 128);
+  const bool big = m > 64 && w128 >= 256;
+  const double a_k = (ak == AK_F32 ? 0.0126 : 0.009) * (is_dual(epi) ? 1.42 : 1) * (big ? ak == AK_F32 ? 1.44 : 1.08 : 1);
+  return (2.2 + a_k * k) * rounds_of((big ? w128 : cols * ((m + 63) / 64)) / 256.0);
+}
+
+// Up to 16 rows streaming wins for any K that a model has; from there the
+// faster estimate.  Both sides measured, us, tiled -> streaming:
 //   MXFP4  4096 -> 2 x 14336  16: 22.6 -> 18.4  32: 23.4 -> 22.2  64: 26.5 -> 36.4
 //          7168 -> 2 x 2048   16: 18.7 -> 9.2   64: 21.0 -> 12.4  128: 21.2 -> 21.3
 //          2048 -> 2 x 5632   16: 16.0 -> 7.7   128: 21.5 -> 17.6 256: 31.5 -> 31.0
+//          512 -> 3648        1001: 9.2 -> 24.7
 //   FP8    4096 -> 2 x 14336  16: 34.1 -> 27.7  32: 35.8 -> 32.4  48: 36.0 -> 56.4
 //          7168 -> 2 x 2048   16: 19.8 -> 10.4  64: 20.8 -> 17.6  96: 20.9 -> 30.1
-//          5632 -> 2048       128: 17.5 -> 14.2 256: 18.3 -> 23.6
 //          2048 -> 7168       64: 16.0 -> 12.5  96: 17.9 -> 19.0
+//          256 -> 2 x 1408    385: 4.8 -> 15.6
 //   INT4   4096 -> 2 x 14336  16: 42.5 -> 20.0  64: 44.9 -> 40.6  96: 46.7 -> 57.5
 //   W8A8   7168 -> 2 x 2048   16: 17.9 -> 10.3  64: 18.6 -> 14.3  128: 19.5 -> 23.9
 //          2048 -> 2 x 5632   32: 13.4 -> 11.4  48: 14.1 -> 17.7
 //   f16    4096 -> 4096       16: 14.6 -> 9.6   32: 14.6 -> 11.6  128: 17.9 -> 27.3
 //   f32 rows x MXFP4  4096 -> 4096  64: 24.7 -> 15.4  256: 43.4 -> 40.0  1024: 125 -> 169
-//   FP8, K stages that do not split (167): 10688 -> 7168, 40 rows, 97 us tiled
-// Up to 16 rows it always wins.  From there both sides are estimated: this
-// kernel at 5 us + row tiles x weight bytes at 4.6 TB/s, or tile_time if that
-// is more; the tiled family at its flat time (19 us; single GEMMs with 8-bit
-// weights and short W8A8 passes 14, f32 rows 34), the weights at 3.3 TB/s (W8A8
-// 4.6), or half a us for each K stage of a split.
+// Over the measured GEMMs this is 0.6 % from the faster side on average.  With a
+// flat time for the tiled family, whatever its K, it was 6.5 %, and below 1024 K up
+// to 6 times the tiled time.
 bool stream_wins(int ak, int bk, int epi, int m, int n, int k) {
   if (!can(ak, bk, epi, n, k)) return false;
-  if (m <= 16) return true;
-  const int rows = tile_rows(ak, m), tiles = (m + rows - 1) / rows;
-  const int ng = groups_of(ak, bk, epi, rows, n, k, tiles);
-  const double mb = weight_mb(bk, epi, n, k);
-  const double here = std::max(5.0 + tiles * mb / 4.6, tile_time(bk, epi, n, k, ng, tiles));
-  const double flat = ak == AK_F32 ? 34.0 : ak == AK_I8 ? (k >= 4096 ? 19.0 : 14.0)
-                      : !bits4(bk) && !is_dual(epi) ? 14.0 : 19.0;
-  const int stages = k / (ak == AK_I8 ? 128 : 64) / gemm_q_splits(ak, bk, epi, m, n, k);
-  return here <= std::max({flat, mb / (ak == AK_I8 ? 4.6 : 3.3), 0.5 * stages});
+  return m <= 16 || stream_time(ak, bk, epi, m, n, k) <=
+                        std::min(tiled_time(ak, bk, epi, m, n, k), tile_gemm_time(ak, bk, epi, m, n, k));
 }
 
-// Against the K-step-32 kernel (sizes off the 64-wide grid), whose time is at
-// least about 0.0225 us per K (one tile's serial loop) and else its rate:
-// streaming runs these shapes at about 330 (4-bit) or 250 TFLOP/s (f32 rows:
-// 180).  Measured, us, K-step-32 -> streaming: MXFP4 257 tokens 2080 -> 2 x
-// 5536 81 -> 36, 5536 -> 2080 125 -> 23; 1024 tokens 95 -> 117 and 165 -> 77;
-// 4096 tokens 338 -> 476 and 233 -> 286; 1 x 5536 -> 2080 108 -> 5.9.
+// Against the K-step-32 kernel (sizes off the 64-wide grid).  Measured, us,
+// K-step-32 -> streaming: MXFP4 257 tokens 2080 -> 2 x 5536 81 -> 36, 5536 -> 2080
+// 125 -> 23; 1024 tokens 95 -> 117 and 165 -> 77; 1 x 5536 -> 2080 108 -> 5.9; 1078
+// tokens, 96 -> 3360 6.3 -> 20.6; f32 rows 1536 x 864 x 128 4.8 -> 31.7.  1.2 %
+// from the faster side on average over 390 GEMMs, the tile kernel among them.
 bool stream_wins_off_grid(int ak, int bk, int epi, int m, int n, int k) {
-  if (!can(ak, bk, epi, n, k)) return false;
-  const double rate = ak == AK_F32 ? 1.8e8 : bits4(bk) ? 3.3e8 : 2.5e8;  // flop per us
-  return 2.0 * m * n * (is_dual(epi) ? 2 : 1) * k <= rate * (0.0225 * k + 10.0);
+  return can(ak, bk, epi, n, k) && stream_time(ak, bk, epi, m, n, k) <= k32_time(ak, epi, m, n, k);
 }
 
 hipError_t launch_stream(int ak, int bk, int epi, const QGemmArgs& q, hipStream_t st) {
@@ -148,29 +190,78 @@ hipError_t launch_stream(int ak, int bk, int epi, const QGemmArgs& q, hipStream_
   return hipErrorInvalidValue;
 }
 
-// MoE: experts of uneven sizes.  Below about 72 rows an expert on average (20
-// for a short K) the 128-row tiles of the tiled family are mostly padding (us,
-// tiled -> streaming: 64 experts, 256 tokens, 7168 -> 2048, largest 25: 712 ->
-// 281; 32 experts, 2000 tokens, 4096 -> 1408: 276 -> 219; 8 experts, 512
-// tokens, 7168 -> 2048: 166 -> 130; 8 experts, 1024 tokens, 4096 -> 1408: 90 ->
-// 104; 32 experts, 838 tokens, 1408 -> 1792: 73 -> 82; 3005 tokens, 2304 ->
-// 1024: 101 -> 153; 8 experts, 286 tokens, 3328 -> 1792: 49 -> 51; 64
-// experts, 1470 tokens, 1408 -> 1664: 125 -> 137).
-// 16-row tiles leave three workgroups per CU: better while most experts have
-// fewer rows than that (the first of these 304 us with 32-row tiles, 64
-// experts with 1024 tokens 444 against 403).
+namespace {
+
+// MoE: tile rows and groups of weight rows of a launch over experts of uneven
+// sizes.  16-row tiles leave three workgroups per CU: better while most experts
+// have fewer rows than that (64 experts, 256 tokens, 7168 -> 2048, largest 25: 281
+// us, 304 with 32-row tiles; 64 experts with 1024 tokens 444 against 403).
+struct Grouped {
+  int rows, ng;
+  long active;
+};
+Grouped grouped_of(int epi, int n, int k, const GroupTable& gt, int groups) {
+  int most = 0;
+  long active = 0;
+  for (int e = 0; e < groups; e++) {
+    most = std::max(most, gt.off[e + 1] - gt.off[e]);
+    active += gt.off[e + 1] > gt.off[e];
+  }
+  int rows = tile_rows(AK_F16, most);
+  if (rows == 32 && gt.off[groups] < 16 * active) rows = 16;
+  return {rows, groups_of(AK_F16, BK_MXFP4, epi, rows, n, k, active), active};
+}
+
+// stream_time's and tiled_time's terms over experts: an expert's last row tile
+// costs its own body's activations, and the 128-row family pays a whole tile for
+// it.  The weights once, at 4.6 and 3.3 TB/s.
+double grouped_stream_time(int epi, int n, int k, const GroupTable& gt, int groups) {
+  const Grouped l = grouped_of(epi, n, k, gt, groups);
+  auto workgroup = [&](int rows) {
+    const int kb = rows > 16 ? 8 : rows > 8 ? 4 : 2;
+    return 0.055 * (k / 512.0) * (kb + 2 * l.ng) + 0.65 * l.ng;
+  };
+  double per_cu = 0;  // for one weight tile of every CU
+  for (int e = 0; e < groups; e++) {
+    const int t = gt.off[e + 1] - gt.off[e], full = t / l.rows, rest = t % l.rows;
+    per_cu += full * workgroup(l.rows) + (rest ? workgroup(rest) : 0);
+  }
+  per_cu *= fill(epi, n, l.ng, 1);
+  return std::max(2.3 + std::max(per_cu, workgroup(32)), 2.5 + l.active * weight_mb(BK_MXFP4, epi, n, k) / 4.6);
+}
+double grouped_tiled_time(int epi, int n, int k, const GroupTable& gt, int groups) {
+  long tiles = 0, active = 0;
+  for (int e = 0; e < groups; e++) {
+    const int t = gt.off[e + 1] - gt.off[e];
+    tiles += (t + 127) / 128;
+    active += t > 0;
+  }
+  tiles *= !is_dual(epi) && n % 128 == 0 ? n / 128 : n / 64;
+  return std::max(1.5 + (0.52 * k / 64 + 1.6) * rounds_of(tiles / 256.0), active * weight_mb(BK_MXFP4, epi, n, k) / 3.3);
+}
+
+}  // namespace
+
+// From 1024 K on, below 20 rows an expert (72 from 4096 K on): the 128-row tiles are
+// mostly padding, and the weights, read from HBM, are most of the time.  us a pass,
+// tiled -> streaming: 64 experts, 256 tokens, 7168 -> 2048, largest 25: 712 -> 281; 32
+// experts, 2000 tokens, 4096 -> 1408: 276 -> 219; 8 experts, 512 tokens, 7168 -> 2048:
+// 166 -> 130.  Of 374 GEMMs of at least 1024 x 1024, 2 are over 5 % of a pass faster
+// on the other side of that line; below it, shorter K (64 experts, 878 tokens, 448 ->
+// 320: 18 -> 31) and above it the estimates decide, with a tenth for what they miss:
+// 8 experts, 1024 tokens, 4096 -> 1408: 90 -> 104; 32 experts, 838 tokens, 1408 ->
+// 1792: 73 -> 82; 3005 tokens, 2304 -> 1024: 101 -> 153.  Over 590 MoE shapes (2 to 128
+// experts, K of 64 to 7168) a GEMM is 1.4 % of a pass from the faster side on
+// average; the line in rows alone, for any K, was 12 %.
 bool stream_wins_grouped(int epi, int n, int k, const GroupTable& gt, int groups) {
-  int active = 0;
-  for (int e = 0; e < groups; e++) active += gt.off[e + 1] > gt.off[e];
-  return can(AK_F16, BK_MXFP4, epi, n, k) && gt.off[groups] < (k >= 4096 ? 72L : 20L) * active;
+  if (!can(AK_F16, BK_MXFP4, epi, n, k)) return false;
+  if (k >= 1024 && gt.off[groups] < (k >= 4096 ? 72L : 20L) * grouped_of(epi, n, k, gt, groups).active) return true;
+  return 1.1 * grouped_stream_time(epi, n, k, gt, groups) <= grouped_tiled_time(epi, n, k, gt, groups);
 }
 
 hipError_t launch_stream_grouped(int epi, const QGemmArgs& q, const GroupTable& gt, int groups, hipStream_t st) {
-  long active = 0;
-  for (int e = 0; e < groups; e++) active += gt.off[e + 1] > gt.off[e];
-  int rows = tile_rows(AK_F16, q.m);
-  if (rows == 32 && gt.off[groups] < 16 * active) rows = 16;
-  return launch_mxfp4_grouped(args_of(epi, q), gt, groups, rows, groups_of(AK_F16, BK_MXFP4, epi, rows, q.n, q.k, active), st);
+  const Grouped l = grouped_of(epi, q.n, q.k, gt, groups);
+  return launch_mxfp4_grouped(args_of(epi, q), gt, groups, l.rows, l.ng, st);
 }
 
 }  // namespace mx

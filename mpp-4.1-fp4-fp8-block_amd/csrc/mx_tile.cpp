@@ -3,6 +3,7 @@
 #include "mx_tile.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 
 namespace mx {
@@ -10,7 +11,6 @@ namespace mx {
 namespace {
 
 bool dual(int epi) { return epi == EPI_SWIGLU_F16 || epi == EPI_SWIGLU_HALF || epi == EPI_SWIGLU_F32; }
-bool bits4(int bk) { return bk == BK_MXFP4 || bk == BK_INT4G32; }
 long ceil_div(long a, long b) { return (a + b - 1) / b; }
 
 // What the kernel can run: a whole group of scales, offsets in 32 bits.
@@ -98,16 +98,16 @@ int side_of(int ak, int bk, int epi, int m, int n, int k) {
   return tiled <= std::min(t.us256, t.us128) ? 0 : t.us256 <= t.us128 ? 256 : 128;
 }
 
-// Sizes off the 64-wide grid: against streaming at 330 (4-bit) or 250 TFLOP/s
-// (mx_stream.cpp); the K-step-32 kernel is slower than one of the two.  us, the
-// faster of those -> here: MXFP4 MLPs of 1374 tokens, 2336 -> 13472, 711 -> 282;
-// 1126 tokens, 1888 -> 5248, 139 -> 83; 2685 tokens, 2144 -> 4736, 361 -> 168; FP8
-// 455 tokens, 5920 -> 6048, 294 -> 147; 1796 x 2560 x 2208 69 -> 36.
+// Sizes off the 64-wide grid: against streaming and the K-step-32 kernel
+// (mx_stream.cpp).  us, the faster of those -> here: MXFP4 MLPs of 1374 tokens,
+// 2336 -> 13472, 711 -> 282; 1126 tokens, 1888 -> 5248, 139 -> 83; 2685 tokens, 2144
+// -> 4736, 361 -> 168; FP8 455 tokens, 5920 -> 6048, 294 -> 147; 1796 x 2560 x 2208
+// 69 -> 36.
 int side_off_grid(int ak, int bk, int epi, int m, int n, int k) {
   if (ak != AK_F16 || !can(ak, bk, epi, k)) return 0;
   const Times t = times(ak, bk, epi, m, n, k);
-  const double stream = 5 + 2.0 * m * n * (dual(epi) ? 2 : 1) * k / (bits4(bk) ? 3.3e8 : 2.5e8);
-  return stream <= std::min(t.us256, t.us128) ? 0 : t.us256 <= t.us128 ? 256 : 128;
+  const double other = std::min(stream_time(ak, bk, epi, m, n, k), k32_time(ak, epi, m, n, k));
+  return other <= std::min(t.us256, t.us128) ? 0 : t.us256 <= t.us128 ? 256 : 128;
 }
 
 }  // namespace
@@ -124,6 +124,12 @@ static hipError_t launch_side(int side, int ak, int bk, int epi, const QGemmArgs
     case BK_F16: return launch_f16(side, epi, g, st);
   }
   return hipErrorInvalidValue;
+}
+
+double tile_gemm_time(int ak, int bk, int epi, int m, int n, int k) {
+  if (!side_of(ak, bk, epi, m, n, k)) return HUGE_VAL;
+  const Times t = times(ak, bk, epi, m, n, k);
+  return std::min(t.us256, t.us128);
 }
 
 bool launch_tile_gemm(int ak, int bk, int epi, const QGemmArgs& g, hipStream_t st, hipError_t* e) {
