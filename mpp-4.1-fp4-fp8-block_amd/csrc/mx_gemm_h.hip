@@ -290,9 +290,11 @@ static hipError_t launch_epi(int epi, const GemmArgs& g, hipStream_t st) {
 hipError_t launch_gemm_h(int bkind, int epi, const GemmArgs& g, hipStream_t st) {
   const int ak = g.a_dtype == MX_DTYPE_F32 ? AK_F32 : AK_F16;
   const QGemmArgs q{g.a, nullptr, g.b0, g.s0, g.b1, g.s1, g.c, nullptr, g.m, g.n, g.k, 0};
-  hipError_t e;
-  if (launch_tile_gemm_off_grid(ak, bkind, epi, q, st, &e)) return e;
-  if (stream_wins_off_grid(ak, bkind, epi, g.m, g.n, g.k)) return launch_stream(ak, bkind, epi, q, st);
+  switch (gemm_kernel(ak, bkind, epi, q)) {
+    case GEMM_STREAM: return launch_stream(ak, bkind, epi, q, st);
+    case GEMM_TILE128: return launch_tile(128, ak, bkind, epi, q, st);
+    case GEMM_TILE256: return launch_tile(256, ak, bkind, epi, q, st);
+  }
   switch (bkind) {
     case BK_F16: return launch_epi<BK_F16>(epi, g, st);
     case BK_MXFP4: return launch_epi<BK_MXFP4>(epi, g, st);

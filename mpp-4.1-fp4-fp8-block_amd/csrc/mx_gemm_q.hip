@@ -1351,24 +1351,13 @@ hipError_t launch_gemm_q_grouped(int epi, const QGemmArgs& g, const GroupTable& 
 
 hipError_t launch_gemm_q(int ak, int bk, int epi, const QGemmArgs& g, hipStream_t st) {
   if (!gemm_q_ok(ak, bk, epi, g.m, g.n, g.k)) return hipErrorInvalidValue;
-  // few tiles (C0): one small tile per CU, operands requested up front
-  // (its scale loads are dwords: planes at a 4-byte boundary)
-  // from 33 rows on (plain GEMMs 17: their 16-row tiles): 16 rows, 1024 -> 2 x
-  // 4096 -> 1024, streaming 4.1 + 5.5 us against 4.7 + 7.5; 64 rows 7.0 + 6.6
-  // against 6.7 + 5.1
-  if (ak == AK_F16 && bk == BK_MXFP4 && small_gemm_ok(epi, g.m, g.n, g.k) && g.m > (is_dual(epi) ? 32 : 16) &&
-      ((reinterpret_cast<uintptr_t>(g.s0) | reinterpret_cast<uintptr_t>(g.s1)) & 3u) == 0)
-    return launch_small_gemm(epi, g, st);
-  if (stream_wins(ak, bk, epi, g.m, g.n, g.k)) return launch_stream(ak, bk, epi, g, st);
-  // about one 64 x 64-channel gate/up tile per CU over a long K (C2): K
-  // split between the waves of a workgroup, no split-K partials
-  if (bk == BK_MXFP4 && kq_gemm_ok(ak, epi, g.m, g.n, g.k) &&
-      ((reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b0) | reinterpret_cast<uintptr_t>(g.b1)) & 15u) == 0 &&
-      ((reinterpret_cast<uintptr_t>(g.s0) | reinterpret_cast<uintptr_t>(g.s1) |
-        (ak == AK_F8X2 ? reinterpret_cast<uintptr_t>(g.a_e8) : 0)) & 3u) == 0)
-    return launch_kq_gemm(ak, epi, g, st);
-  hipError_t e;
-  if (launch_tile_gemm(ak, bk, epi, g, st, &e)) return e;
+  switch (gemm_kernel(ak, bk, epi, g)) {
+    case GEMM_SMALL: return launch_small_gemm(epi, g, st);
+    case GEMM_STREAM: return launch_stream(ak, bk, epi, g, st);
+    case GEMM_KQ: return launch_kq_gemm(ak, epi, g, st);
+    case GEMM_TILE128: return launch_tile(128, ak, bk, epi, g, st);
+    case GEMM_TILE256: return launch_tile(256, ak, bk, epi, g, st);
+  }
   const int s = gemm_q_splits(ak, bk, epi, g.m, g.n, g.k);
   if (s > 1 && !g.ws) return hipErrorInvalidValue;
   if (ak == AK_I8) {

@@ -43,7 +43,7 @@ enum BKind : int {
 // Activation encodings of the small-M GEMM family (mx_gemm_q.hip).
 enum AKind : int {
   AK_F16 = 0,      // f16 [M][K]
-  AK_F32 = 1,      // f32 [M][K] (rounded to f16 for the MFMA)
+  AK_F32 = 1,      // f32 [M][K] (two f16 terms for the MFMA)
   AK_I8 = 2,       // int8 [M][K] + f32 per-row (token) scale [M]
   AK_F8X2 = 3,     // two FP8 E4M3 terms + E8M0 scales per 64 K (the F8X2 layout below)
 };
@@ -109,12 +109,19 @@ struct QGemmArgs {
   const void* pf = nullptr;
   int pf_rows = 0, pf_row_bytes = 0;
 };
-// Prefill tile GEMM (mx_gemm_tile.h, choice in mx_tile.cpp): launched, with its
-// status in *e, where it is faster than the 64-K-stage family (off_grid: than
-// the kernels for sizes off the 64-wide grid); false where it is not.
-bool launch_tile_gemm(int akind, int bkind, int epi, const QGemmArgs& g, hipStream_t st, hipError_t* e);
-bool launch_tile_gemm_off_grid(int akind, int bkind, int epi, const QGemmArgs& g, hipStream_t st, hipError_t* e);
-// Estimate of a GEMM there, us; infinite where launch_tile_gemm does not take it.
+// Which kernel a GEMM runs on (mx_route.cpp): for sizes that gemm_q_ok takes one
+// of the first five or GEMM_Q (the 64-K-stage family), else streaming, the tile
+// kernel or GEMM_H (the K-step-32 kernel).
+enum GemmKernel : int { GEMM_SMALL, GEMM_STREAM, GEMM_KQ, GEMM_TILE128, GEMM_TILE256, GEMM_Q, GEMM_H };
+int gemm_kernel(int akind, int bkind, int epi, const QGemmArgs& g);
+// Prefill tile GEMM (mx_gemm_tile.h, choice in mx_tile.cpp).  tile_side: its tile,
+// 256 or 128, or 0 where the 64-K-stage family (off_grid: streaming or the
+// K-step-32 kernel) is faster.
+int tile_side(int akind, int bkind, int epi, int m, int n, int k);
+int tile_side_off_grid(int akind, int bkind, int epi, int m, int n, int k);
+bool tile_aligned(int bkind, const QGemmArgs& g);
+hipError_t launch_tile(int side, int akind, int bkind, int epi, const QGemmArgs& g, hipStream_t st);
+// Estimate of a GEMM there, us; infinite where tile_side is 0.
 double tile_gemm_time(int akind, int bkind, int epi, int m, int n, int k);
 // Weight-streaming GEMM (mx_gemm_stream.h, choice in mx_stream.cpp): any n,
 // k % 32 == 0, few rows (or sizes off the tile grid).  stream_wins: against

@@ -21,12 +21,6 @@ bool can(int ak, int bk, int epi, int k) {
   return k % 32 == 0 && k >= 256;
 }
 
-bool aligned(int bk, const QGemmArgs& g) {
-  const uintptr_t p = reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b0) | reinterpret_cast<uintptr_t>(g.b1);
-  const uintptr_t s = reinterpret_cast<uintptr_t>(g.s0) | reinterpret_cast<uintptr_t>(g.s1);
-  return p % 16 == 0 && s % (bk == BK_MXFP4 ? 1 : bk == BK_INT4G32 ? 2 : 4) == 0;
-}
-
 // Times of the three kernels, us, per K stage (64 K; int8 128) and for the
 // launch with its first loads and last stores.  The 256-tile runs one workgroup
 // a CU: a full round of 256 costs `full` a stage (the card's matrix rate), one
@@ -61,6 +55,8 @@ Times times(int ak, int bk, int epi, int m, int n, int k) {
   return {t128, us256, ak == AK_I8 ? us256 + 1 : 7 + kt * std::max(r.own128, r.round128 * t128 / 256)};
 }
 
+}  // namespace
+
 // Tile side, 0 where the 128-row tiled family is the faster one.  By the times
 // above, fitted to 200 GEMMs of 256 to 4096 rows (5 formats, 4 MLP sizes), which
 // they get right to 10 % or where the sides differ less.  Some of them, us,
@@ -76,7 +72,7 @@ Times times(int ak, int bk, int epi, int m, int n, int k) {
 //          14336 -> 4096       1000 rows 78 / 175         2048 139 / 181         4096 262 / 200
 // Below 150 tiles of 128 the split-K launches keep more CUs busy than either
 // tile does; from there to 192 they pay for a second launch and the partials.
-int side_of(int ak, int bk, int epi, int m, int n, int k) {
+int tile_side(int ak, int bk, int epi, int m, int n, int k) {
   if (!can(ak, bk, epi, k)) return 0;
   const Times t = times(ak, bk, epi, m, n, k);
   if (t.t128 < 150) return 0;
@@ -103,16 +99,20 @@ int side_of(int ak, int bk, int epi, int m, int n, int k) {
 // 2336 -> 13472, 711 -> 282; 1126 tokens, 1888 -> 5248, 139 -> 83; 2685 tokens, 2144
 // -> 4736, 361 -> 168; FP8 455 tokens, 5920 -> 6048, 294 -> 147; 1796 x 2560 x 2208
 // 69 -> 36.
-int side_off_grid(int ak, int bk, int epi, int m, int n, int k) {
+int tile_side_off_grid(int ak, int bk, int epi, int m, int n, int k) {
   if (ak != AK_F16 || !can(ak, bk, epi, k)) return 0;
   const Times t = times(ak, bk, epi, m, n, k);
   const double other = std::min(stream_time(ak, bk, epi, m, n, k), k32_time(ak, epi, m, n, k));
   return other <= std::min(t.us256, t.us128) ? 0 : t.us256 <= t.us128 ? 256 : 128;
 }
 
-}  // namespace
+bool tile_aligned(int bk, const QGemmArgs& g) {
+  const uintptr_t p = reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b0) | reinterpret_cast<uintptr_t>(g.b1);
+  const uintptr_t s = reinterpret_cast<uintptr_t>(g.s0) | reinterpret_cast<uintptr_t>(g.s1);
+  return p % 16 == 0 && s % (bk == BK_MXFP4 ? 1 : bk == BK_INT4G32 ? 2 : 4) == 0;
+}
 
-static hipError_t launch_side(int side, int ak, int bk, int epi, const QGemmArgs& g, hipStream_t st) {
+hipError_t launch_tile(int side, int ak, int bk, int epi, const QGemmArgs& g, hipStream_t st) {
   using namespace tile;
   if (ak == AK_I8) return launch_i8(epi, g, st);
   switch (bk) {
@@ -127,21 +127,9 @@ static hipError_t launch_side(int side, int ak, int bk, int epi, const QGemmArgs
 }
 
 double tile_gemm_time(int ak, int bk, int epi, int m, int n, int k) {
-  if (!side_of(ak, bk, epi, m, n, k)) return HUGE_VAL;
+  if (!tile_side(ak, bk, epi, m, n, k)) return HUGE_VAL;
   const Times t = times(ak, bk, epi, m, n, k);
   return std::min(t.us256, t.us128);
-}
-
-bool launch_tile_gemm(int ak, int bk, int epi, const QGemmArgs& g, hipStream_t st, hipError_t* e) {
-  const int side = aligned(bk, g) ? side_of(ak, bk, epi, g.m, g.n, g.k) : 0;
-  if (side) *e = launch_side(side, ak, bk, epi, g, st);
-  return side != 0;
-}
-
-bool launch_tile_gemm_off_grid(int ak, int bk, int epi, const QGemmArgs& g, hipStream_t st, hipError_t* e) {
-  const int side = aligned(bk, g) ? side_off_grid(ak, bk, epi, g.m, g.n, g.k) : 0;
-  if (side) *e = launch_side(side, ak, bk, epi, g, st);
-  return side != 0;
 }
 
 }  // namespace mx

@@ -1,20 +1,10 @@
 """Which kernel a GEMM runs on (host logic, no GPU): the launchers' rules against
 GEMMs where one side was measured at least 1.2 times as fast as the other."""
-import ctypes
-
 import pytest
 
-import mxfp4hip as M
-
-F16, F32, I8 = 0, 1, 2                                             # activations
-W_F16, MXFP4, E4M3, INT8, INT4, W_I8 = 0, 1, 2, 4, 5, 6            # weights
-STORE_F32, STORE_F16, SWIGLU_F16, SWIGLU_HALF, SWIGLU_F32 = range(5)
-
-
-def _fn(name, restype=ctypes.c_bool):
-    f = getattr(M.load(), name)
-    f.restype = restype
-    return f
+import test_gpu_kernels as G
+from gemm_route import (E4M3, F16, F32, I8, INT4, INT8, MXFP4, STORE_F16, STORE_F32, STORE_I32, SWIGLU_F16,
+                        SWIGLU_F32, W_F16, W_I8, mlp_routes, moe_streams, route)
 
 
 # (activations, weights, epilogue, m, n, k, streaming is faster): us streaming / tiled
@@ -46,7 +36,7 @@ ON_GRID = [
 
 @pytest.mark.parametrize("ak,bk,epi,m,n,k,stream", ON_GRID)
 def test_streaming_where_it_is_faster(ak, bk, epi, m, n, k, stream):
-    assert _fn("_ZN2mx11stream_winsEiiiiii")(ak, bk, epi, m, n, k) is stream
+    assert (route(ak, bk, epi, m, n, k) == "stream") is stream
 
 
 # us streaming / the K-step-32 kernel
@@ -66,7 +56,7 @@ OFF_GRID = [
 
 @pytest.mark.parametrize("ak,bk,epi,m,n,k,stream", OFF_GRID)
 def test_streaming_off_the_grid(ak, bk, epi, m, n, k, stream):
-    assert _fn("_ZN2mx20stream_wins_off_gridEiiiiii")(ak, bk, epi, m, n, k) is stream
+    assert (route(ak, bk, epi, m, n, k) == "stream") is stream
 
 
 @pytest.mark.parametrize("counts,n,k,stream", [
@@ -78,7 +68,19 @@ def test_streaming_off_the_grid(ak, bk, epi, m, n, k, stream):
     ([94] * 32, 1024, 2304, False),          # 153 / 101
 ])
 def test_grouped_streaming_where_it_is_faster(counts, n, k, stream):
-    table = (ctypes.c_int * 262)()           # off[257], then the strides
-    for e, c in enumerate(counts):
-        table[e + 1] = table[e] + c
-    assert _fn("_ZN2mx19stream_wins_groupedEiiiRKNS_10GroupTableEi")(SWIGLU_F16, n, k, table, len(counts)) is stream
+    assert moe_streams(counts, SWIGLU_F16, n, k) is stream
+
+
+def test_gpu_cases_reach_their_kernels():
+    for a, b, m, n, k, kernel in G.MATMULS:
+        assert route(a, b, STORE_F32, m, n, k) == kernel, (a, b, m, n, k)
+    for fmt, t, h, i, up, down in G.MLPS:
+        assert mlp_routes(fmt, t, h, i) == (up, down), (fmt, t, h, i)
+    for m, n, k in G.I8:
+        assert route(I8, W_I8, STORE_I32, m, n, k) == "tile256"
+    for _, t, h, i in G.E8M0_255:
+        assert mlp_routes(0, t, h, i) == ("q", "q")
+    for t, h, i, up, down in G.INT4_SCALES:
+        assert mlp_routes(G.M.WFMT_INT4, t, h, i) == (up, down)
+    counts, h, i = G.MOE_Q
+    assert not moe_streams(counts, SWIGLU_F16, i, h) and not moe_streams(counts, STORE_F16, h, i)
