@@ -93,9 +93,9 @@ def test_format_mlp_small(dev, wfmt, T):
 
 @pytest.mark.parametrize("wfmt", MLP_FMTS)
 def test_format_mlp_deep_ragged(dev, wfmt):
-    """Gate/up on the deep ring (K = 1024: 16 stages; 2 x 32 tiles), a
-    ragged second token tile, and per-workgroup start stages that wrap
-    (7 (w / 8) mod 16)."""
+    """Gate/up of the 8-bit formats on the deep ring (K = 1024: 16 stages; 2 x 32
+    tiles), a ragged second token tile, and per-workgroup start stages that wrap
+    (7 (w / 8) mod 16); INT4 and the down GEMMs stream."""
     d = MlpData(dev, 130, 1024, 2048, seed=53 + wfmt, wfmt=wfmt)
     got = run_fmt(dev, d, wfmt)
     rel, cos = O.mlp_error(got, oracle_fmt(d, wfmt))
@@ -131,11 +131,9 @@ def test_config3_formats(dev, wfmt):
 
 def test_int4_scale_planes_4_byte_aligned(dev):
     """INT4 scale planes at a 4-byte offset against 16-byte aligned ones,
-    same output bits.  The gate/up GEMM (224 tiles, deep ring) copies its
-    32 KB of f16 scales per workgroup to LDS by dword DMA either way; the
-    down GEMM (2-slot ring, scales not in LDS) loads a B chunk's scales
-    with one 16-byte load per lane from aligned planes and one scale per
-    stage from shifted ones."""
+    same output bits, at 32 tokens: both GEMMs stream, whose scale copy goes
+    by 16-byte DMA from aligned planes and by 8-byte pieces from shifted ones
+    (test_gpu_kernels.py has the 64-K-stage family and the tile kernel)."""
     T, H, I = 32, 4096, 14336
     d = MlpData(dev, T, H, I, seed=41, wfmt=M.WFMT_INT4)
     ref = run_fmt(dev, d, M.WFMT_INT4)

@@ -28,8 +28,8 @@ def check(got, ref, tol=TOL, cos_min=COS, what=""):
     assert rel <= tol and cos >= cos_min, (what, rel, cos)
 
 
-# Shapes cover both tile widths (n % 128, n % 64), split K (few tiles, long
-# K), ragged M and the K-step-32 fallback kernel (k % 64 != 0).
+# Few rows and few weight rows, ragged M, long K and k % 64 != 0 (streaming and
+# the few-tile kernel; the 64-K-stage family from (300, 64, 2048) on).
 @pytest.mark.parametrize("m,n,k", [(1, 128, 256), (7, 192, 512), (64, 128, 1024), (100, 256, 512),
                                    (300, 64, 2048), (5, 64, 96)])
 def test_mxfp4_matmul(dev, m, n, k):
@@ -48,8 +48,7 @@ def test_mxfp4_matmul(dev, m, n, k):
         dc.free()
 
 
-# (96, 128, 512): the tiled family; (40, 96, 160): k % 64 != 0, the
-# K-step-32 kernel.  An f32 A goes in as two f16 terms (hi + lo), so both A
+# (96, 128, 512): K in steps of 64; (40, 96, 160): k % 64 != 0.  An f32 A goes in as two f16 terms (hi + lo), so both A
 # types are held to f32 accumulation error (mpp_mlp_f_h_f_n128 multiplies
 # f32 x half, MPPMLPKernels.metal:164-173); rounding A to f16 instead
 # measured ~3e-3 of rms.
@@ -441,8 +440,8 @@ def _check_nonfinite_pattern(got, ref, what):
 @pytest.mark.parametrize("which", ["gate", "down"])
 def test_e8m0_endpoints_tiled_paths(dev, variant, which):
     """E8M0 bytes 255 (+inf in the reference, MXFP4Kernels.metal:26-29) and
-    0 (0.0) on the tiled small-M GEMM (fused, T > 16) and on the
-    dequant-to-half path: non-finite outputs where the oracle has them,
+    0 (0.0) on the streaming gate/up and the few-tile down GEMM (fused, T > 16;
+    test_gpu_kernels.py has the 64-K-stage family) and on the dequant-to-half path: non-finite outputs where the oracle has them,
     tolerance elsewhere."""
     T, H, I = 40, 512, 1024
     d = MlpData(dev, T, H, I, seed=131 + variant)

@@ -158,10 +158,9 @@ def test_moe_gemm_large_groups(dev):
 
 
 def test_moe_gemm_long_k_chunk_scales(dev):
-    """Grouped gate/up GEMM at H=7168: its E8M0 scales (28 KB per workgroup)
-    do not fit the LDS copy, so each lane loads a B chunk's scales with one
-    8-byte load.  Sampled tokens against the oracle; the same planes copied
-    to a 4-byte offset take the per-stage byte loads and give the same bits."""
+    """Grouped gate/up GEMM at H=7168 with 207 rows over three experts: streaming
+    (test_gpu_kernels.py has the 64-K-stage family).  Sampled tokens against the
+    oracle; the same planes copied to a 4-byte offset give the same bits."""
     counts, H, I = [40, 0, 150, 17], 7168, 256
     d = MoeData(dev, counts, H, I, seed=93)
     got = d.run()

@@ -4,8 +4,9 @@ The reference runs its MXFP4 rows whenever hidden % 32 == 0 and
 intermediate % 32 == 0 (main.swift:1043), and its matmul tiles guard
 column < n (MXFP4Kernels.metal:98), so any n works there.  The library's
 64-K-stage GEMM family needs multiples of 64; the other shapes go to the
-K-step-32 kernel with a masked N tail.  Every shape here is checked
-against the oracle (dequantize-then-accumulate, float64) within the
+weight-streaming, tile or K-step-32 kernel with a masked N tail, at these
+sizes mostly to streaming (test_gpu_kernels.py has the others).  Every shape
+here is checked against the oracle (dequantize-then-accumulate, float64) within the
 BASELINE tolerance.
 """
 import numpy as np
@@ -43,8 +44,8 @@ def oracle_mlp(d, variant, rows):
 
 # (5, 96, 160): neither size % 64, T below the MFMA tile; (40, 1056, 2080)
 # and (130, 544, 1120): % 32 only, ragged M tiles; (8, 192, 320): % 64 but not
-# % 128 with few tokens (64-K-stage family, not the decode GEMV); (3, 32, 64):
-# the smallest MXFP4 block shape.
+# % 128 with few tokens (streaming, not the decode GEMV); (3, 32, 64): the
+# smallest MXFP4 block shape (K-step-32 kernel).
 SHAPES = [(5, 96, 160), (40, 1056, 2080), (130, 544, 1120), (8, 192, 320), (3, 32, 64)]
 
 
@@ -119,7 +120,7 @@ def test_gemm_f16_any_n(dev, m, n, k):
 
 @pytest.mark.parametrize("wfmt", [M.WFMT_FP8_E4M3, M.WFMT_FP8_E5M2, M.WFMT_INT8, M.WFMT_INT4])
 def test_format_mlp_shape_domain(dev, wfmt):
-    """The weight-format rows at % 32 shapes run on the K-step-32 kernel."""
+    """The weight-format rows at % 32 shapes (few tokens: streaming)."""
     T, H, I = 5, 96, 160
     d = MlpData(dev, T, H, I, seed=400 + wfmt, wfmt=wfmt)
     out = dev.alloc(T * H * 2)

@@ -1,6 +1,6 @@
-"""The prefill tile GEMM: edges of its 128- and 256-wide tiles, the shortest K
-and K stages that leave a remainder of its ring, every weight format, E8M0 byte
-255.  References are float64 products of the dequantized operands; f32 sums of
+"""The prefill tile GEMM: edges of its 128-wide tiles (and one whole 256-wide
+product), K stages that leave a remainder of its ring, every weight format, E8M0
+byte 255; test_gpu_kernels.py has the 256-wide tile's edges and formats.  References are float64 products of the dequantized operands; f32 sums of
 k terms in another order stay within sqrt(k) 2^-23 of the products' norm, far
 below the 1e-5 of rms used for f32 results; an f16 store is the f32 one rounded."""
 import numpy as np
@@ -13,9 +13,10 @@ from test_gpu_stream import E2M1, close, mxfp4
 pytestmark = pytest.mark.gpu
 
 
-# (m, n, k) on the 128- and 256-wide tiles: whole, one row or 64 channels past
-# a tile, one row short, a single 256-K ring; then K that ends a quarter, half or
-# three quarters into a group of four stages, or in the middle of a stage
+# (m, n, k) on the 128-wide tile (4096 x 4096 x 512: the 256-wide one; K = 256: the
+# 64-K-stage family): whole, one row or 64 channels past a tile, one row short; then
+# K that ends a quarter, half or three quarters into a group of four stages, or in
+# the middle of a stage
 SHAPES = [(1024, 4096, 256), (1281, 8128, 768), (1000, 4160, 512), (4096, 4096, 512), (4095, 4160, 768), (4097, 2112, 1280),
           (1281, 8128, 320), (4095, 4160, 384), (4095, 4160, 448), (1500, 5013, 288), (4095, 4131, 416), (4097, 2099, 1440)]
 
