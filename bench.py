@@ -63,9 +63,10 @@ def roofline_block(bound, work, us, peak_key, kernel):
             "peak_dtype": peak_key, "frac": round(rate / peak, 4), "kernel": kernel, "kernel_us": round(us, 3)}
 
 
-# The step kernels of the library's MLP forwards (mx_mlp_kernel_name /
-# mx_fmt_mlp_kernel_name) that a roofline may be taken on, by what bounds
-# them.  Anything else (quantize / split prologues, the byte-255 fix-up
+# The steps of the library's MLP forwards (mx_mlp_kernel_name /
+# mx_fmt_mlp_kernel_name: named for sizes and formats, gemm_q_* on the grid of
+# 64 channels x 64 K and gemm_h_* off it, whichever kernel the library chose
+# for the rows) that a roofline may be taken on, by what bounds them.  Anything else (quantize / split prologues, the byte-255 fix-up
 # passes, the standalone SwiGLU) is never the roofline kernel.
 GEMM_GATE_UP = {"gemm_q_mxfp4_gate_up_swiglu", "gemm_q_mxfp4_gate_up_swiglu_half", "gemm_h_mxfp4_gate_up_swiglu",
                 "gemm_h_mxfp4_gate_up_swiglu_half", "gemm_q_scaled_gate_up_swiglu",

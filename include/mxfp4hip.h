@@ -245,8 +245,10 @@ int mx_mlp_benchmark(mx_ctx* ctx, int variant, const mx_mlp_config* cfg, const v
                      const mx_mlp_weights* sets, int n_sets, void* out, int warmup,
                      int iterations, int use_graph, double* seconds_out, double* kernel_us_out,
                      int* n_kernels_out);
-/* Name of kernel `index` of the forward that `variant` runs at shape `cfg`
- * (for the per-kernel times); NULL past the last kernel. */
+/* Name of step `index` of the forward that `variant` runs at shape `cfg` (for
+ * the per-kernel times); NULL past the last one.  A GEMM step is named for its
+ * sizes and formats, not for the kernel chosen for its number of rows:
+ * gemm_q_* on the grid of 64 channels x 64 K, gemm_h_* off it. */
 const char* mx_mlp_kernel_name(int variant, const mx_mlp_config* cfg, int index);
 
 /* ---- MoE grouped experts ------------------------------------------------------ */
@@ -304,8 +306,8 @@ int mx_fmt_mlp_benchmark(mx_ctx* ctx, int wfmt, const mx_mlp_config* cfg, const 
                          const mx_mlp_weights* sets, int n_sets, void* out, int warmup,
                          int iterations, int use_graph, double* seconds_out, double* kernel_us_out,
                          int* n_kernels_out);
-/* Name of kernel `index` of the format forward at shape `cfg`; NULL past the
- * last kernel. */
+/* Name of step `index` of the format forward at shape `cfg` (as
+ * mx_mlp_kernel_name); NULL past the last one. */
 const char* mx_fmt_mlp_kernel_name(int wfmt, const mx_mlp_config* cfg, int index);
 
 /* ---- synthetic data (main.swift:2785-2842) ---------------------------------- */

@@ -92,13 +92,13 @@ int ensure_ws(mx_ctx* c, size_t bytes) {
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // Split-K partial bytes of a GEMM that the 64-K-stage family takes (0 when
-// the shape goes to the K-step-32 kernel, which does not split K).
+// the shape is off its grid: the kernels for those do not split K).
 size_t q_ws(int ak, int bk, int epi, int m, int n, int k) {
   return mx::gemm_q_ok(ak, bk, epi, m, n, k) ? mx::gemm_q_ws_bytes(ak, bk, epi, m, n, k) : 0;
 }
 
-// One GEMM of an MLP: the 64-K-stage family when the shape fits it, else the
-// K-step-32 kernel (any n, k % 32 == 0).
+// One GEMM of an MLP: sizes on the 64-K-stage family's grid, or any n and
+// k % 32 == 0; gemm_kernel says which kernel runs.
 hipError_t launch_mlp_gemm(int ak, int bk, int epi, const mx::QGemmArgs& q, hipStream_t st) {
   if (mx::gemm_q_ok(ak, bk, epi, q.m, q.n, q.k)) return mx::launch_gemm_q(ak, bk, epi, q, st);
   mx::GemmArgs g{q.a, ak == mx::AK_F32 ? MX_DTYPE_F32 : MX_DTYPE_F16, q.b0, q.s0, q.b1, q.s1, q.c, q.m, q.n, q.k};
@@ -143,9 +143,10 @@ bool gemv_ok(const mx_mlp_config* cfg) {
 }
 
 // Which kernels a forward runs (shared by the launcher and the name query).
-// PATH_GEMM_H: the fused (or reference-row) MLP at shapes the 64-K-stage
-// family does not take (hidden or intermediate % 64 != 0): both GEMMs on the
-// K-step-32 kernel.
+// PATH_GEMM_Q / PATH_GEMM_H: the fused (or reference-row) MLP on the 64-K-stage
+// family's grid and off it (hidden or intermediate % 64 != 0).  A path names
+// the sizes, as the step names do; which kernel a GEMM runs on is gemm_kernel's
+// choice (mx_route.cpp).
 // PATH_W4A4: stage-major scale planes (the 256 x 256 kernels, whose down
 // epilogue recomputes byte-255 outputs itself); PATH_W4A4_REF: the
 // reference-layout kernels plus a separate byte-255 pass.
@@ -268,7 +269,7 @@ int build_mlp_steps(mx_ctx* c, int variant, const mx_mlp_config* cfg, const void
     steps.push_back({"gemv_mxfp4_gate_up_swiglu", [=] { return mx::launch_gemv_mxfp4(1, gu, st); }});
     steps.push_back({"gemv_mxfp4_down", [=] { return mx::launch_gemv_mxfp4(0, dn, st); }});
   } else if (path == PATH_GEMM_H || path == PATH_REFROW_H) {
-    // hidden or intermediate % 64 != 0: both GEMMs on the K-step-32 kernel
+    // hidden or intermediate % 64 != 0: both GEMMs off the 64-wide grid
     uint16_t* mid = reinterpret_cast<uint16_t*>(ws + s.mid);
     const bool ref = path == PATH_REFROW_H;
     const int e_gu = ref ? mx::EPI_SWIGLU_HALF : mx::EPI_SWIGLU_F16;
@@ -612,8 +613,7 @@ static int check_gemm(mx_ctx* c, int m, int n, int k, const void* a, const void*
   return MX_OK;
 }
 
-// One GEMM through the small-M family when the shape fits it (k % 64),
-// else through the K-step-32 kernel.
+// One GEMM on the 64-K-stage family's grid (n and k % 64) or off it.
 // ws_off: bytes of the workspace the caller already uses (kept in front of
 // the split-K partials).
 static int run_gemm(mx_ctx* c, const void* a, int a_dtype, int bk, const void* b, const void* scales,
@@ -931,8 +931,8 @@ int mx_mlp_benchmark(mx_ctx* c, int variant, const mx_mlp_config* cfg, const voi
 
 // ---- MoE: grouped experts ---------------------------------------------------------
 // Two grouped launches for all experts: the decode GEMV when every expert has
-// at most 16 tokens, else the small-M GEMM family (one tile grid per expert
-// in blockIdx.z).  Expert e owns token rows [off[e], off[e+1]).
+// at most 16 tokens, else the streaming kernel or the 64-K-stage family (one
+// tile grid per expert in blockIdx.y or .z).  Expert e owns token rows [off[e], off[e+1]).
 static int build_moe_steps(mx_ctx* c, const mx_mlp_config* cfg, int n_experts, const int* counts,
                            const void* x, const mx_mlp_weights* w, void* out, std::vector<Step>& steps) {
   if (int rc = check_mlp_cfg(c, MX_MLP_FUSED, cfg)) return rc;

@@ -3,10 +3,11 @@
 //
 //   C[m][n] = sum_k A[m][k] * W[n][k]   (epilogue: store, SwiGLU, row scales)
 //
-// Bound: the f16 matrix cores.  4096 tokens, 4096 -> 2 x 14336 -> 4096 with MXFP4
-// weights run at 1.45 PFLOP/s, what a large f16 matrix product reaches on this
-// card; per K stage a CU's four SIMDs need 2048 clocks for a 256-tile's MFMAs
-// and the rest has to fit beneath them:
+// Bound: the f16 matrix cores, busy 83 to 89 %.  4096 tokens, 4096 -> 2 x 14336 ->
+// 4096 with MXFP4 weights run at 1.45 PFLOP/s; on a card where they run at 1.33,
+// library products of 16384 reach 1.23 in f16 and 1.31 in bf16.  Per K stage a
+// CU's four SIMDs need 2048 clocks for a 256-tile's MFMAs and the rest has to fit
+// beneath them:
 //   LDS read    a wave owns 128 x 64 of the tile (T = 128: 64 x 64), 192 rows
 //               of fragments for 8192 outputs; four waves of 128 x 128 read a
 //               third less but leave one wave a SIMD, whose waits then show
@@ -14,7 +15,10 @@
 //   L2 -> LDS   a CU takes in 50 to 70 bytes a ns by DMA, whatever the ring's
 //               depth or the cache policy: 40 KB a stage for the 256-tile
 //               (0.6 us of 1.06), 20 KB for a quarter of the work with the
-//               128-tile (0.35 of 0.41, its bound).
+//               128-tile (0.35 of 0.41, its bound).  With int8 activations
+//               (64 KB stages of 128 K, two slots) the matrix cores are busy 52 %
+//               at 28 bytes a ns: waves wait at the barrier for a stage's last
+//               loads, and four slots of half a stage were no faster.
 //   widening    in registers, one k-step ahead of its MFMAs, spread between
 //               them (sched_group_barrier; 1017 -> 1000 us for the MLP).
 // The weights stay in their stored form up to the registers: a 64-K stage of a
