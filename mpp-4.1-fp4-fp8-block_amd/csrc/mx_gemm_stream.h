@@ -45,6 +45,7 @@
 #include <type_traits>
 
 #include "mx_device.h"
+#include "mx_dma.h"
 #include "mx_internal.h"
 #include "mx_stream.h"
 #include "mx_widen.h"
@@ -85,20 +86,6 @@ constexpr int wait_count(int xi, int wl, int d, int dw, int ps, int phase) {
   if (phase) return a;
   const int b = after(i - dw * ps, true);
   return a < b ? a : b;
-}
-
-typedef __attribute__((address_space(3))) uint32_t* lds_u32;
-extern "C" __device__ void llvm_amdgcn_raw_buffer_load_lds_s(v4i rsrc, lds_u32 lds, int size, int voffset, int soffset,
-                                                              int offset, int aux) __asm("llvm.amdgcn.raw.buffer.load.lds");
-
-__device__ __forceinline__ v4i rsrc_of(const void* base, uint32_t bytes) {
-  const uint64_t a = reinterpret_cast<uint64_t>(base);
-  v4i r;
-  r[0] = (int)(uint32_t)a;
-  r[1] = (int)(uint32_t)(a >> 32);
-  r[2] = (int)bytes;
-  r[3] = 0x00020000;
-  return r;
 }
 
 __device__ __forceinline__ void dma16(const void* src, void* lds) { __builtin_amdgcn_global_load_lds(src, lds, 16, 0, 0); }
@@ -155,7 +142,7 @@ __device__ __forceinline__ void tile(const Args& g, int m0, int nt, const Lds& l
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int K = g.k, N = g.n, KB = K / 32;
-  const bool dual = is_dual(g.epi);
+  const bool dual = is_gate_up(g.epi);
   const int PB = dual ? 8 : 16;                     // output channels per group
   const int n0 = nt * NG * PB;
   const int row_b = K / 8 * b_bits(BK);             // bytes of a weight row
@@ -218,7 +205,7 @@ __device__ __forceinline__ void tile(const Args& g, int m0, int nt, const Lds& l
   constexpr int SW = CH < 16 ? CH - 1 : 15;  // chunk swizzle of a row
   const int a_row = K * a_elem(AK);
   const uint8_t* ab = reinterpret_cast<const uint8_t*>(g.a) + (size_t)m0 * a_row;
-  const v4i ars = rsrc_of(ab, (uint32_t)T * (uint32_t)a_row);
+  const v4i ars = rsrc_of<false>(ab, (uint32_t)T * (uint32_t)a_row);
   int a_off[XI];
 #pragma unroll
   for (int i = 0; i < XI; i++) {
@@ -245,7 +232,7 @@ __device__ __forceinline__ void tile(const Args& g, int m0, int nt, const Lds& l
     unroll<0, XI>([&](auto qq) {
       constexpr int q = decltype(qq)::value, U = decltype(u)::value;
       uint8_t* dst = piece(std::integral_constant<int, U * MT + q / XP>{}) + (q % XP) * 1024;
-      llvm_amdgcn_raw_buffer_load_lds_s(ars, (lds_u32)dst, 16, a_off[q] + o, 0, 0, 0);
+      buffer_dma16(ars, dst, a_off[q] + o);
     });
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -553,7 +540,7 @@ __global__ __launch_bounds__(64 * kNW) void k_stream(Args g, typename std::condi
     g.c = reinterpret_cast<uint8_t*>(g.c) + (size_t)t0 * g.n * 2;
     g.b0 += e * gt.b_stride;
     g.s0 += e * gt.s_stride;
-    if (is_dual(g.epi)) {
+    if (is_gate_up(g.epi)) {
       g.b1 += e * gt.b_stride;
       g.s1 += e * gt.s_stride;
     }
@@ -573,7 +560,7 @@ __global__ __launch_bounds__(64 * kNW) void k_stream(Args g, typename std::condi
 template <int AK, int BK, int NG, int MAXR, bool GROUPED>
 hipError_t launch_ng(const Args& g0, const GroupTable* gt, int groups, hipStream_t st) {
   Args g = g0;
-  const int pb = (is_dual(g.epi) ? 8 : 16) * NG;
+  const int pb = (is_gate_up(g.epi) ? 8 : 16) * NG;
   g.m_tiles = (g.m + MAXR - 1) / MAXR;
   g.n_tiles = (g.n + pb - 1) / pb;
   const dim3 grid((unsigned)((g.n_tiles + 7) / 8 * 8 * g.m_tiles), groups);

@@ -40,6 +40,7 @@
 #include <type_traits>
 
 #include "mx_device.h"
+#include "mx_dma.h"
 #include "mx_internal.h"
 #include "mx_tile.h"
 #include "mx_widen.h"
@@ -47,8 +48,6 @@
 namespace mx {
 namespace tile {
 
-constexpr bool is_dual(int epi) { return epi == EPI_SWIGLU_F16 || epi == EPI_SWIGLU_HALF || epi == EPI_SWIGLU_F32; }
-constexpr bool bits4(int bk) { return bk == BK_MXFP4 || bk == BK_INT4G32; }
 // bytes of a weight row per stage (64 K; int8 activations 128)
 constexpr int rb_of(int bk) { return bk == BK_F16 || bk == BK_I8 ? 128 : bits4(bk) ? 32 : 64; }
 constexpr int slots_of(int bk) { return rb_of(bk) == 128 ? 2 : bits4(bk) ? 4 : 3; }
@@ -72,23 +71,10 @@ __device__ __forceinline__ int swz(int row) {
   return (row / RPL) % C;
 }
 
-typedef __attribute__((address_space(3))) uint32_t* lds_u32;
-extern "C" __device__ void llvm_amdgcn_raw_buffer_load_lds_b(v4i rsrc, lds_u32 lds, int size, int voffset, int soffset,
-                                                              int offset, int aux) __asm("llvm.amdgcn.raw.buffer.load.lds");
-__device__ __forceinline__ v4i rsrc_of(const void* base, uint32_t bytes) {
-  const uint64_t a = reinterpret_cast<uint64_t>(base);
-  v4i r;
-  r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)a);
-  r[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32));
-  r[2] = __builtin_amdgcn_readfirstlane((int)bytes);
-  r[3] = 0x00020000;
-  return r;
-}
-
 template <int AK, int BK, int EPI, int T>
 __global__ __launch_bounds__(T * 2, 2) void k_tile(QGemmArgs g, int n_tiles) {
   static_assert(T == 256 || T == 128, "tile side");
-  constexpr bool DUAL = is_dual(EPI), S4 = bits4(BK);
+  constexpr bool DUAL = is_gate_up(EPI), S4 = bits4(BK);
   constexpr int KS = AK == AK_I8 ? 128 : 64, RA = 128, RB = rb_of(BK), NS = slots_of(BK);
   constexpr int NW = T / 32;
   constexpr int SLOT = T * (RA + RB), BO = T * RA;
@@ -119,10 +105,10 @@ __global__ __launch_bounds__(T * 2, 2) void k_tile(QGemmArgs g, int n_tiles) {
 
   // ---- DMA: wave w moves tile rows [32 w, +32) of A and of B, whole rows of
   // a stage per instruction; rows past the end read as zero
-  const v4i ars = rsrc_of(reinterpret_cast<const uint8_t*>(g.a) + (size_t)m0 * a_row, (uint32_t)min(T, M - m0) * a_row);
+  const v4i ars = rsrc_of<true>(reinterpret_cast<const uint8_t*>(g.a) + (size_t)m0 * a_row, (uint32_t)min(T, M - m0) * a_row);
   const int bfirst = DUAL ? n0 + (wave & (NW / 2 - 1)) * RW : n0 + wave * RW;
   const uint8_t* bsrc = reinterpret_cast<const uint8_t*>(DUAL && wave >= NW / 2 ? g.b1 : g.b0) + (size_t)min(bfirst, N - 1) * b_row;
-  const v4i brs = rsrc_of(bsrc, (uint32_t)max(0, min(RW, N - bfirst)) * (uint32_t)b_row);
+  const v4i brs = rsrc_of<true>(bsrc, (uint32_t)max(0, min(RW, N - bfirst)) * (uint32_t)b_row);
   // (K % 64 == 32: the upper half of the last stage reads as zero too)
   constexpr int kPast = 0x40000000;  // past every row range
   const int half_stage = K % KS ? KT - 1 : -1;
@@ -154,12 +140,10 @@ __global__ __launch_bounds__(T * 2, 2) void k_tile(QGemmArgs g, int n_tiles) {
     const int ao = k < KT ? k * RA : kPast, bo = k < KT ? k * RB : kPast, up = k == half_stage ? kPast : 0;
 #pragma unroll
     for (int q = 0; q < NA; q++)
-      llvm_amdgcn_raw_buffer_load_lds_b(ars, (lds_u32)(s + (wave * NA + q) * 1024), 16,
-                                        a_off[q] + ao + (a_up[q] & up), 0, 0, 0);
+      buffer_dma16(ars, s + (wave * NA + q) * 1024, a_off[q] + ao + (a_up[q] & up));
 #pragma unroll
     for (int q = 0; q < NBI; q++)
-      llvm_amdgcn_raw_buffer_load_lds_b(brs, (lds_u32)(s + BO + (wave * NBI + q) * 1024), 16,
-                                        b_off[q] + bo + (b_up[q] & up), 0, 0, 0);
+      buffer_dma16(brs, s + BO + (wave * NBI + q) * 1024, b_off[q] + bo + (b_up[q] & up));
   };
 
   // ---- fragments
@@ -461,7 +445,7 @@ template <int AK, int BK, int EPI, int T>
 hipError_t launch_one(const QGemmArgs& g0, hipStream_t st) {
   QGemmArgs g = g0;
   g.tiles_m = (g.m + T - 1) / T;
-  const int per = is_dual(EPI) ? T / 2 : T, n_tiles = (g.n + per - 1) / per;
+  const int per = is_gate_up(EPI) ? T / 2 : T, n_tiles = (g.n + per - 1) / per;
   hipLaunchKernelGGL((k_tile<AK, BK, EPI, T>), dim3(g.tiles_m * n_tiles), dim3(2 * T), 0, st, g, n_tiles);
   return hipGetLastError();
 }

@@ -70,6 +70,10 @@ enum Epi : int {
   EPI_SWIGLU_F8X2 = 6,   // dual B: mid = silu(g) * u in f32, stored as F8X2 (c data, c_e8 scales)
 };
 
+// Two weight matrices, SwiGLU of their sums to f16 or f32.
+constexpr bool is_gate_up(int epi) { return epi == EPI_SWIGLU_F16 || epi == EPI_SWIGLU_HALF || epi == EPI_SWIGLU_F32; }
+constexpr bool bits4(int bk) { return bk == BK_MXFP4 || bk == BK_INT4G32; }
+
 struct GemmArgs {
   const void* a;  int a_dtype;            // f16 or f32 [M][K]
   const void* b0; const void* s0;         // weights + scales (matrix 0)

@@ -11,8 +11,6 @@ using namespace stream;
 
 namespace {
 
-bool bits4(int bk) { return bk == BK_MXFP4 || bk == BK_INT4G32; }
-
 // Bytes of a workgroup's scale copy.
 size_t scale_bytes(int bk, int ng, int k) {
   return bits4(bk) ? (size_t)16 * ng * (k / 32) * (bk == BK_INT4G32 ? 2 : 1) : 0;
@@ -20,7 +18,7 @@ size_t scale_bytes(int bk, int ng, int k) {
 
 // Megabytes of weight codes of the launch.
 double weight_mb(int bk, int epi, int n, int k) {
-  return (double)n * (is_dual(epi) ? 2 : 1) * k * (bits4(bk) ? 0.5 : bk == BK_F16 ? 2.0 : 1.0) * 1e-6;
+  return (double)n * (is_gate_up(epi) ? 2 : 1) * k * (bits4(bk) ? 0.5 : bk == BK_F16 ? 2.0 : 1.0) * 1e-6;
 }
 
 // Rows of a tile.  32 at most: larger tiles leave one workgroup per CU, and a
@@ -32,7 +30,7 @@ int tile_rows(int ak, int m) { return m <= 4 && ak != AK_I8 ? 4 : m <= 8 ? 8 : m
 // Workgroups of a launch over the CUs of its fullest XCD (32 CUs each, weight
 // tiles dealt out round robin, `tiles` row tiles to each).
 double fill(int epi, int n, int ng, long tiles) {
-  const int per = (is_dual(epi) ? 8 : 16) * ng, nt = (n + per - 1) / per;
+  const int per = (is_gate_up(epi) ? 8 : 16) * ng, nt = (n + per - 1) / per;
   return (nt + 7) / 8 * tiles / 32.0;
 }
 
@@ -58,7 +56,7 @@ double tile_time(int bk, int epi, int n, int k, int ng, long tiles) {
 // pass (256 groups) 11.4 / 14.4 / -; 16 tokens, 2048 -> 7168 (448) 6.1 / 5.4 /
 // 7.4; 1 token, 2080 -> 2 x 5536 (692) 7.9 / 8.4 / 9.3.
 int groups_of(int ak, int bk, int epi, int rows, int n, int k, long tiles) {
-  const int per = is_dual(epi) ? 8 : 16, most = bk == BK_F16 ? 2 : 4;
+  const int per = is_gate_up(epi) ? 8 : 16, most = bk == BK_F16 ? 2 : 4;
   int ng = 1;
   for (int c = 2; c <= most && scale_bytes(bk, c, k) <= kScales; c *= 2) {
     if (rows == (ak == AK_F32 ? 16 : 32)) {
@@ -77,7 +75,7 @@ Args args_of(int epi, const QGemmArgs& q) {
 
 // What the kernel can run: its scale copy, and offsets in 32 bits.
 bool can(int ak, int bk, int epi, int n, int k) {
-  if (k % 32 || k > (1 << 20) || (size_t)n * (is_dual(epi) ? 2 : 1) > (1u << 30) || scale_bytes(bk, 1, k) > kScales) return false;
+  if (k % 32 || k > (1 << 20) || (size_t)n * (is_gate_up(epi) ? 2 : 1) > (1u << 30) || scale_bytes(bk, 1, k) > kScales) return false;
   const bool store = epi == EPI_STORE_F32 || epi == EPI_STORE_F16;
   if (ak == AK_I8) return bk == BK_I8 && k % 128 == 0 && (store || epi == EPI_STORE_I32 || epi == EPI_SWIGLU_F32);
   if (ak == AK_F32) return (bk == BK_F16 || bk == BK_MXFP4) && store;
@@ -119,11 +117,11 @@ static double tiled_time(int ak, int bk, int epi, int m, int n, int k) {
                  : bk == BK_F16 ? Rate{1.6, 0.43, 1.35, 1.65} : bk == BK_INT4G32 ? Rate{1.75, 0.635, 1.65, 1.65}
                  : bk == BK_MXFP4 ? Rate{1.5, 0.52, 1.6, 2.0} : Rate{3.7, 0.5, 0.85, 0.35};
   const int s = gemm_q_splits(ak, bk, epi, m, n, k);
-  const long tiles = (long)((m + 127) / 128) * (!is_dual(epi) && n % 128 == 0 ? n / 128 : n / 64);
+  const long tiles = (long)((m + 127) / 128) * (!is_gate_up(epi) && n % 128 == 0 ? n / 128 : n / 64);
   double t = r.start + (r.stage * k / (ak == AK_I8 ? 128 : 64) / s + r.round) * rounds_of(tiles * s / 256.0);
-  if (s > 1) t += r.split + 0.47 * s * (is_dual(epi) ? 2 : 1) * m * n * 4e-6 + (ak == AK_I8 ? 0 : 0.27 * s);
+  if (s > 1) t += r.split + 0.47 * s * (is_gate_up(epi) ? 2 : 1) * m * n * 4e-6 + (ak == AK_I8 ? 0 : 0.27 * s);
   // MXFP4 gate/up from HBM: a tenth more (76 rows, 3072 -> 2 x 3072: 17.0 us)
-  if (bk == BK_MXFP4 && is_dual(epi)) t *= 1.1;
+  if (bk == BK_MXFP4 && is_gate_up(epi)) t *= 1.1;
   // one 64 x 64-channel gate/up tile per CU (34 rows, 2560 -> 2 x 12416: 14.1
   // us against 26.0 streaming; 512 rows, 7168 -> 2 x 2048: 31)
   if (bk == BK_MXFP4 && kq_gemm_ok(ak, epi, m, n, k)) t = std::min(t, 4.7 + 0.0037 * k);
@@ -136,7 +134,7 @@ static double tiled_time(int ak, int bk, int epi, int m, int n, int k) {
 double k32_time(int ak, int epi, int m, int n, int k) {
   const long cols = (n + 63) / 64, w128 = cols * ((m + 127) / 128);
   const bool big = m > 64 && w128 >= 256;
-  const double a_k = (ak == AK_F32 ? 0.0126 : 0.009) * (is_dual(epi) ? 1.42 : 1) * (big ? ak == AK_F32 ? 1.44 : 1.08 : 1);
+  const double a_k = (ak == AK_F32 ? 0.0126 : 0.009) * (is_gate_up(epi) ? 1.42 : 1) * (big ? ak == AK_F32 ? 1.44 : 1.08 : 1);
   return (2.2 + a_k * k) * rounds_of((big ? w128 : cols * ((m + 63) / 64)) / 256.0);
 }
 
@@ -236,7 +234,7 @@ double grouped_tiled_time(int epi, int n, int k, const GroupTable& gt, int group
     tiles += (t + 127) / 128;
     active += t > 0;
   }
-  tiles *= !is_dual(epi) && n % 128 == 0 ? n / 128 : n / 64;
+  tiles *= !is_gate_up(epi) && n % 128 == 0 ? n / 128 : n / 64;
   return std::max(1.5 + (0.52 * k / 64 + 1.6) * rounds_of(tiles / 256.0), active * weight_mb(BK_MXFP4, epi, n, k) / 3.3);
 }
 

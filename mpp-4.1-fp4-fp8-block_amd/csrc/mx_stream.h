@@ -19,8 +19,6 @@ struct Args {
   int m_tiles, n_tiles;             // set by the launcher
 };
 
-constexpr bool is_dual(int epi) { return epi == EPI_SWIGLU_F16 || epi == EPI_SWIGLU_HALF || epi == EPI_SWIGLU_F32; }
-
 // rows: activation rows of a tile (4, 8, 16 or 32), ng: groups of 16 weight rows of a workgroup (1, 2 or 4)
 hipError_t launch_mxfp4(const Args& g, int rows, int ng, hipStream_t st);
 hipError_t launch_f32_mxfp4(const Args& g, int rows, int ng, hipStream_t st);

@@ -10,7 +10,6 @@ namespace mx {
 
 namespace {
 
-bool dual(int epi) { return epi == EPI_SWIGLU_F16 || epi == EPI_SWIGLU_HALF || epi == EPI_SWIGLU_F32; }
 long ceil_div(long a, long b) { return (a + b - 1) / b; }
 
 // What the kernel can run: a whole group of scales, offsets in 32 bits.
@@ -47,7 +46,7 @@ struct Times {
   double us256, us128;
 };
 Times times(int ak, int bk, int epi, int m, int n, int k) {
-  const long n_rows = (long)n * (dual(epi) ? 2 : 1);
+  const long n_rows = (long)n * (is_gate_up(epi) ? 2 : 1);
   const long t256 = ceil_div(m, 256) * ceil_div(n_rows, 256), t128 = ceil_div(m, 128) * ceil_div(n_rows, 128);
   const double kt = k / (ak == AK_I8 ? 128.0 : 64.0), last = (t256 % 256) / 256.0;
   const Rates& r = rates(ak, bk);
@@ -88,7 +87,7 @@ int tile_side(int ak, int bk, int epi, int m, int n, int k) {
   // tiles and K are faster here: 1024 rows, 2048 -> 2 x 2048 41.1 / 39.5, 768 rows,
   // 2048 -> 2 x 2304 39.1 / 38.2, 900 rows, 2048 -> 2 x 1792 39.7 / 38.7, 512 rows, 2048
   // -> 2 x 3584 36.6 / 36.0, K = 1024 level.
-  if (bk == BK_MXFP4 && !dual(epi) && t.t128 >= 192 && t.t128 <= 256 && kt <= 32) return 0;
+  if (bk == BK_MXFP4 && !is_gate_up(epi) && t.t128 >= 192 && t.t128 <= 256 && kt <= 32) return 0;
   const Rates& r = rates(ak, bk);
   const double tiled = t.t128 < 192 ? 17 + kt * 0.32 : t.t128 <= 256 ? 7 + kt * r.deep : r.start + kt * r.tiled * t.t128 / 256;
   return tiled <= std::min(t.us256, t.us128) ? 0 : t.us256 <= t.us128 ? 256 : 128;
