@@ -84,10 +84,6 @@ bool can(int ak, int bk, int epi, int n, int k) {
 
 }  // namespace
 
-// Rounds that workgroups filling the chip x times take: between x (they start
-// as others end) and whole ones.
-static double rounds_of(double x) { return std::max(1.0, 0.55 * x + 0.45 * std::ceil(x)); }
-
 // Time of a launch, us: 2 for it, its first loads and its sums, and for each
 // workgroup of a CU 0.055 a step and KB and 0.65 (4-bit weights) to 1.5 a group
 // of weight rows for its scales and its outputs; two share a CU, further ones
@@ -107,21 +103,33 @@ double stream_time(int ak, int bk, int epi, int m, int n, int k) {
   return std::max(2.5 + tiles * weight_mb(bk, epi, n, k) / 4.6, r.start + std::max(0.3, rounds * wg));
 }
 
-// Time of the 64-K-stage family, us (1700 GEMMs of its sizes, half within 8 %,
-// nine in ten within 25 %): rounds of 256 workgroups at 0.5 a K stage (f32
-// activations 1.35), a split's partials at 2.1 MB a us and their sum, the weights
-// at 3.3 TB/s (W8A8 4.6).
+// Rounds that workgroups filling the chip x > 1 times take: between x (they start
+// as others end) and whole ones.
+static double rounds_of(double x) { return x > 1 ? (x + std::ceil(x)) / 2 : x; }
+
+// Time of `stages` K stages of the 64-K-stage family, us: a workgroup's own
+// latency a stage, or where more, the rate of a full chip.  Narrow: 64 weight rows
+// a workgroup, else 128.  Fitted to 2400 GEMMs with tiled_time, half of them
+// within 6 %, nine in ten within 19 %.
+static double stages_time(int ak, int bk, bool narrow, double stages, double workgroups) {
+  struct Rate { double own, full; };
+  struct Rates { double start; Rate narrow, wide; };
+  const Rates r = ak == AK_F32 ? Rates{3.5, {1.21, 1.11}, {1.48, 1.79}} : ak == AK_I8 ? Rates{5.6, {0.49, 0.7}, {0.49, 0.7}}
+                  : bk == BK_F16 ? Rates{2.8, {0.28, 0.38}, {0.5, 0.62}} : bk == BK_INT4G32 ? Rates{3.5, {0.42, 0.41}, {0.65, 0.67}}
+                  : bk == BK_MXFP4 ? Rates{3.25, {0.41, 0.37}, {0.56, 0.56}} : Rates{4.7, {0.3, 0.39}, {0.52, 0.55}};
+  const Rate& w = narrow ? r.narrow : r.wide;
+  return r.start + stages * std::max(w.own, w.full * rounds_of(workgroups / 256));
+}
+
+// Time of the 64-K-stage family, us: its stages, a split's partials at 2.3 MB a us
+// and their sum, or the weights at 3.3 TB/s (W8A8 4.6).
 static double tiled_time(int ak, int bk, int epi, int m, int n, int k) {
-  struct Rate { double start, stage, round, split; };
-  const Rate r = ak == AK_F32 ? Rate{0.7, 1.35, 3.05, 2.5} : ak == AK_I8 ? Rate{1.6, 0.49, 3.9, 2.5}
-                 : bk == BK_F16 ? Rate{1.6, 0.43, 1.35, 1.65} : bk == BK_INT4G32 ? Rate{1.75, 0.635, 1.65, 1.65}
-                 : bk == BK_MXFP4 ? Rate{1.5, 0.52, 1.6, 2.0} : Rate{3.7, 0.5, 0.85, 0.35};
   const int s = gemm_q_splits(ak, bk, epi, m, n, k);
-  const long tiles = (long)((m + 127) / 128) * (!is_gate_up(epi) && n % 128 == 0 ? n / 128 : n / 64);
-  double t = r.start + (r.stage * k / (ak == AK_I8 ? 128 : 64) / s + r.round) * rounds_of(tiles * s / 256.0);
-  if (s > 1) t += r.split + 0.47 * s * (is_gate_up(epi) ? 2 : 1) * m * n * 4e-6 + (ak == AK_I8 ? 0 : 0.27 * s);
-  // MXFP4 gate/up from HBM: a tenth more (76 rows, 3072 -> 2 x 3072: 17.0 us)
-  if (bk == BK_MXFP4 && is_gate_up(epi)) t *= 1.1;
+  const bool narrow = !is_gate_up(epi) && (n % 128 != 0 || (bk == BK_MXFP4 && n / 128 < 16));  // as wide_tiles of mx_gemm_q.hip
+  const long tiles = (long)((m + 127) / 128) * (is_gate_up(epi) || narrow ? n / 64 : n / 128);
+  double t = stages_time(ak, bk, narrow, (double)k / (ak == AK_I8 ? 128 : 64) / s, (double)tiles * s);
+  const bool bytes = bk == BK_E4M3 || bk == BK_E5M2 || bk == BK_INT8 || bk == BK_I8;
+  if (s > 1) t += (bytes ? 0.4 : 1.5) + 0.25 * s + 0.43 * s * (is_gate_up(epi) ? 2 : 1) * m * n * 4e-6;
   // one 64 x 64-channel gate/up tile per CU (34 rows, 2560 -> 2 x 12416: 14.1
   // us against 26.0 streaming; 512 rows, 7168 -> 2 x 2048: 31)
   if (bk == BK_MXFP4 && kq_gemm_ok(ak, epi, m, n, k)) t = std::min(t, 4.7 + 0.0037 * k);
@@ -129,13 +137,17 @@ static double tiled_time(int ak, int bk, int epi, int m, int n, int k) {
 }
 
 // Time of the K-step-32 kernel, us, of 64 columns x 64 rows a workgroup, or 128
-// rows from 256 such workgroups on (390 GEMMs off the grid, 2 to 4000 rows, half
-// within 12 %).
+// rows from 256 such workgroups on: a serial loop over K of 0.009 to 0.017 us a K
+// (f32 rows 0.0126 to 0.02), the same for sizes that look alike.  Taken at 1.3
+// times the low end, the choice between it, streaming and the tile kernel is 1.2 %
+// from the fastest on average over 490 GEMMs off the grid (2 to 4000 rows); with
+// a fixed rate for streaming instead of its estimate it was 10.5 %.
 double k32_time(int ak, int epi, int m, int n, int k) {
   const long cols = (n + 63) / 64, w128 = cols * ((m + 127) / 128);
   const bool big = m > 64 && w128 >= 256;
-  const double a_k = (ak == AK_F32 ? 0.0126 : 0.009) * (is_gate_up(epi) ? 1.42 : 1) * (big ? ak == AK_F32 ? 1.44 : 1.08 : 1);
-  return (2.2 + a_k * k) * rounds_of((big ? w128 : cols * ((m + 63) / 64)) / 256.0);
+  const double a_k = (ak == AK_F32 ? 0.0164 : 0.0117) * (is_gate_up(epi) ? 1.42 : 1) * (big ? ak == AK_F32 ? 1.44 : 1.08 : 1);
+  const double x = (big ? w128 : cols * ((m + 63) / 64)) / 256.0;
+  return (2.9 + a_k * k) * std::max(1.0, 0.6 * x + 0.4 * std::ceil(x));
 }
 
 // Up to 16 rows streaming wins for any K that a model has; from there the
@@ -153,7 +165,7 @@ double k32_time(int ak, int epi, int m, int n, int k) {
 //          2048 -> 2 x 5632   32: 13.4 -> 11.4  48: 14.1 -> 17.7
 //   f16    4096 -> 4096       16: 14.6 -> 9.6   32: 14.6 -> 11.6  128: 17.9 -> 27.3
 //   f32 rows x MXFP4  4096 -> 4096  64: 24.7 -> 15.4  256: 43.4 -> 40.0  1024: 125 -> 169
-// Over the measured GEMMs this is 0.6 % from the faster side on average.  With a
+// Over the measured GEMMs this is 0.5 % from the faster side on average.  With a
 // flat time for the tiled family, whatever its K, it was 6.5 %, and below 1024 K up
 // to 6 times the tiled time.
 bool stream_wins(int ak, int bk, int epi, int m, int n, int k) {
@@ -165,8 +177,7 @@ bool stream_wins(int ak, int bk, int epi, int m, int n, int k) {
 // Against the K-step-32 kernel (sizes off the 64-wide grid).  Measured, us,
 // K-step-32 -> streaming: MXFP4 257 tokens 2080 -> 2 x 5536 81 -> 36, 5536 -> 2080
 // 125 -> 23; 1024 tokens 95 -> 117 and 165 -> 77; 1 x 5536 -> 2080 108 -> 5.9; 1078
-// tokens, 96 -> 3360 6.3 -> 20.6; f32 rows 1536 x 864 x 128 4.8 -> 31.7.  1.2 %
-// from the faster side on average over 390 GEMMs, the tile kernel among them.
+// tokens, 96 -> 3360 6.3 -> 20.6; f32 rows 1536 x 864 x 128 4.8 -> 31.7.
 bool stream_wins_off_grid(int ak, int bk, int epi, int m, int n, int k) {
   return can(ak, bk, epi, n, k) && stream_time(ak, bk, epi, m, n, k) <= k32_time(ak, epi, m, n, k);
 }
@@ -234,8 +245,9 @@ double grouped_tiled_time(int epi, int n, int k, const GroupTable& gt, int group
     tiles += (t + 127) / 128;
     active += t > 0;
   }
-  tiles *= !is_gate_up(epi) && n % 128 == 0 ? n / 128 : n / 64;
-  return std::max(1.5 + (0.52 * k / 64 + 1.6) * rounds_of(tiles / 256.0), active * weight_mb(BK_MXFP4, epi, n, k) / 3.3);
+  const bool narrow = !is_gate_up(epi) && n % 128 != 0;
+  tiles *= is_gate_up(epi) || narrow ? n / 64 : n / 128;
+  return std::max(stages_time(AK_F16, BK_MXFP4, narrow, k / 64.0, (double)tiles), active * weight_mb(BK_MXFP4, epi, n, k) / 3.3);
 }
 
 }  // namespace
@@ -246,15 +258,16 @@ double grouped_tiled_time(int epi, int n, int k, const GroupTable& gt, int group
 // experts, 2000 tokens, 4096 -> 1408: 276 -> 219; 8 experts, 512 tokens, 7168 -> 2048:
 // 166 -> 130.  Of 374 GEMMs of at least 1024 x 1024, 2 are over 5 % of a pass faster
 // on the other side of that line; below it, shorter K (64 experts, 878 tokens, 448 ->
-// 320: 18 -> 31) and above it the estimates decide, with a tenth for what they miss:
+// 320: 18 -> 31) and above it the estimates decide, with a fifth for what they miss:
 // 8 experts, 1024 tokens, 4096 -> 1408: 90 -> 104; 32 experts, 838 tokens, 1408 ->
-// 1792: 73 -> 82; 3005 tokens, 2304 -> 1024: 101 -> 153.  Over 590 MoE shapes (2 to 128
-// experts, K of 64 to 7168) a GEMM is 1.4 % of a pass from the faster side on
-// average; the line in rows alone, for any K, was 12 %.
+// 1792: 73 -> 82; 886 tokens, 1408 -> 1664: 67 -> 76; 3005 tokens, 2304 -> 1024: 101
+// -> 153.  Over 590 MoE shapes (2 to 128 experts, K of 64 to 7168) a GEMM is 1.5 %
+// of a pass from the faster side on average; the line in rows alone, for any K,
+// was 12 %.
 bool stream_wins_grouped(int epi, int n, int k, const GroupTable& gt, int groups) {
   if (!can(AK_F16, BK_MXFP4, epi, n, k)) return false;
   if (k >= 1024 && gt.off[groups] < (k >= 4096 ? 72L : 20L) * grouped_of(epi, n, k, gt, groups).active) return true;
-  return 1.1 * grouped_stream_time(epi, n, k, gt, groups) <= grouped_tiled_time(epi, n, k, gt, groups);
+  return 1.2 * grouped_stream_time(epi, n, k, gt, groups) <= grouped_tiled_time(epi, n, k, gt, groups);
 }
 
 hipError_t launch_stream_grouped(int epi, const QGemmArgs& q, const GroupTable& gt, int groups, hipStream_t st) {

@@ -26,7 +26,7 @@ FP8_INT = [M.WFMT_FP8_E4M3, M.WFMT_FP8_E5M2, M.WFMT_INT8, M.WFMT_INT4]
 # tiles, a ragged last row tile, n off 32 and off 64.  tile256: ragged in both
 # directions, K in the middle of a stage and of a group of four.
 MATMULS = [(a, b, *s) for a in (R.F16, R.F32) for b in (R.MXFP4, R.W_F16)
-           for s in ((130, 801, 160, "h"), (1500, 2075, 96, "h"))]
+           for s in ((600, 801, 160, "h"), (1500, 2075, 96, "h"))]
 MATMULS += [(R.F32, b, 2048, 2080, 1056, "h") for b in (R.MXFP4, R.W_F16)]
 MATMULS += [(R.F16, R.MXFP4, 2049, 7040, 288, "tile256"), (R.F16, R.MXFP4, 1500, 10691, 352, "tile256"),
             (R.F16, R.W_F16, 1500, 10691, 352, "tile256"), (R.F16, R.W_F16, 4096, 4096, 512, "tile256"),
